@@ -3,15 +3,26 @@
 // Contract (tools/q4k_ref.py:67-92, RTL order src/glm_matmul_q4k.v:261-270): for each
 // output (m, n) the weight row is dequantised exactly and
 //     acc = f32(acc + f32(x[m][k] * w[n][k]))     for k = 0 .. K-1, in order,
-// then y = bf16_RNE(acc).  One lane owns one output row and walks K sequentially.  Q4_K with
-// K <= 32768 runs k_gemv_ref_q4k (row blocks in registers, activations staged once as fp32),
-// Q8_0 / F16 / BF16 with K a multiple of 64 k_gemv_ref_reg and Q6_K with K a multiple of 512
-// k_gemv_ref_q6k (the same for their blocks), all with aligned pointers; larger K, other K and
-// unaligned pointers run k_gemv_ref, whose 64 rows per workgroup are staged 256
-// weights at a time through LDS so the global reads stay coalesced, with a last stage of fewer
-// weights for K that is a multiple of the type's block but not of 256 (Q8_0: 32; F16 / BF16:
-// any K).  The library is compiled with -ffp-contract=off, so the multiply and the add below
-// are two separately rounded ops.
+// then y = bf16_RNE(acc).  The library is compiled with -ffp-contract=off, so the multiply and
+// the add are two separately rounded ops.
+//
+// What bounds it: the K dependent adds of one output.  They cannot be split or reordered, and a
+// dependent v_add_f32 takes 8.3 cycles on this part (measured), 21 us for K = 6144 at 2.4 GHz.
+// A workgroup has chain waves, whose lanes own one output (m, row) each and add its products in
+// k order, and four producer waves that dequantise for them: a producer lane takes a run (16
+// consecutive weights of one row) and writes to LDS, four consecutive k per 16-B slot, neighbouring
+// rows in neighbouring slots.  What it writes depends on what is scarce:
+//   * One or two activation rows: the products x * w, so that the chain is a read and four adds per
+//     four k (the read hides behind the adds' latency; 10 cycles per k measured).
+//   * More: the weights, with the stage's activations as fp32 beside them, and the chain multiplies.
+//     A chain wave then takes 15 cycles per k, but the producers, whose products of eight rows took
+//     28 cycles per k, write each weight once (M = 8 at 6144 x 6144: 82 -> 47 us).
+// Stages of KS values of k go through a ring of three LDS buffers with one workgroup barrier per
+// stage: in interval t the producers write stage t and the chains add stage t - 2, reading ahead
+// into stage t - 1, which is complete already.
+// Measured (Q4_K, 6144 x 6144): M = 1 79 -> 23.5 us, M = 8 169 -> 45 us against one wave per 64 rows
+// doing everything; the other types within a few us of these.
+// Any K (the last stage may be partial), any 2-byte aligned pointers (unaligned 16-B loads).
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -19,186 +30,21 @@ namespace aipu {
 
 namespace {
 
-constexpr int kRows = 64;      // rows per workgroup (one wave)
+constexpr int kRows = 64;      // rows per workgroup of the fp32-weight kernel (one wave)
 constexpr int kMC = 8;         // activation rows per pass (blockIdx.y walks the rest)
-constexpr int kStageW = 256;   // weights per stage
+constexpr int kStageW = 256;   // weights per stage of the fp32-weight kernel
 
-template <int TYPE>
-struct Stage {
-    static constexpr int bytes = (int)row_bytes(TYPE, kStageW);    // per row per stage
-    static constexpr int u16 = bytes / 2;
-    static constexpr int stride = u16 + ((u16 & 1) ? 0 : 1);        // odd stride in u16 words
-};
-
-// Dequantise weight k (0..255) of the row's current stage, reading the staged bytes.
-// Q4_K: tools/q4k_ref.py:45-60.  Computed per 32-weight sub-block by the caller.
-template <int TYPE>
-__device__ __forceinline__ void stage_mac(const uint8_t* rb, const float (*xs)[kStageW], int mcnt, float* acc,
-                                          int kn) {
-    if constexpr (TYPE == T_Q4_K) {
-        const uint16_t* h = (const uint16_t*)rb;
-        const float d = f16_to_f32(h[0]);
-        const float dm = f16_to_f32(h[1]);
-        uint32_t s[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            s[i] = (uint32_t)rb[4 + 4 * i] | ((uint32_t)rb[5 + 4 * i] << 8) | ((uint32_t)rb[6 + 4 * i] << 16) |
-                   ((uint32_t)rb[7 + 4 * i] << 24);
-        const uint8_t* qs = rb + 16;
-        for (int j = 0; j < 8; ++j) {
-            uint32_t sc, m;
-            q4k_scale_min(j, s[0], s[1], s[2], sc, m);
-            const float D = d * (float)sc;
-            const float Mn = dm * (float)m;
-            const int g = j >> 1, hi = j & 1;
-            for (int l = 0; l < 32; ++l) {
-                const uint32_t q = hi ? (qs[32 * g + l] >> 4) : (qs[32 * g + l] & 0xFu);
-                const float w = q4k_weight_exact(D, Mn, q);
-                const int k = 32 * j + l;
-                for (int mm = 0; mm < kMC; ++mm) {
-                    if (mm < mcnt) {
-                        const float p = xs[mm][k] * w;
-                        acc[mm] = acc[mm] + p;
-                    }
-                }
-            }
-        }
-    } else if constexpr (TYPE == T_Q6_K) {
-        // ql[128] qh[64] int8 sc[16] fp16 d  (tools/q4k_ref.py:105-124)
-        const float d = f16_to_f32((uint32_t)rb[208] | ((uint32_t)rb[209] << 8));
-        for (int k = 0; k < 256; ++k) {
-            const int h = k >> 7, t = (k >> 5) & 3, l = k & 31;
-            const uint32_t qlb = rb[64 * h + l + 32 * (t & 1)];
-            const uint32_t nib = t < 2 ? (qlb & 0xFu) : (qlb >> 4);
-            const uint32_t code = nib | ((((uint32_t)rb[128 + 32 * h + l]) >> (2 * t)) & 3u) << 4;
-            const float ds = d * (float)(int8_t)rb[192 + (k >> 4)];
-            const float w = ds * (float)((int)code - 32);
-            for (int mm = 0; mm < kMC; ++mm) {
-                if (mm < mcnt) {
-                    const float p = xs[mm][k] * w;
-                    acc[mm] = acc[mm] + p;
-                }
-            }
-        }
-    } else if constexpr (TYPE == T_Q8_0) {
-        // up to 8 blocks of fp16 d | int8 qs[32]  (tools/q4k_ref.py:126-129)
-        for (int b = 0; b < kn / 32; ++b) {
-            const uint8_t* p8 = rb + 34 * b;
-            const float d = f16_to_f32((uint32_t)p8[0] | ((uint32_t)p8[1] << 8));
-            for (int i = 0; i < 32; ++i) {
-                const float w = d * (float)(int8_t)p8[2 + i];
-                const int k = 32 * b + i;
-                for (int mm = 0; mm < kMC; ++mm) {
-                    if (mm < mcnt) {
-                        const float p = xs[mm][k] * w;
-                        acc[mm] = acc[mm] + p;
-                    }
-                }
-            }
-        }
-    } else {  // F16 / BF16 passthrough
-        const uint16_t* h = (const uint16_t*)rb;
-        for (int k = 0; k < kn; ++k) {
-            const float w = TYPE == T_F16 ? f16_to_f32(h[k]) : bf16_to_f32(h[k]);
-            for (int mm = 0; mm < kMC; ++mm) {
-                if (mm < mcnt) {
-                    const float p = xs[mm][k] * w;
-                    acc[mm] = acc[mm] + p;
-                }
-            }
-        }
-    }
+// ---------------------------------------------------------------- runs of 16 weights
+// 16 bytes at any 2-byte aligned address (global memory takes unaligned 16-B loads).
+typedef uint32_t u32x4_u2 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 load16_u2(const void* p) {
+    const u32x4_u2 v = *(const u32x4_u2*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// Slot gathering (MoE): blockIdx.z = slot z reads weight matrix sel[z] of the `_exps`
-// stack at W + sel[z]*wstride when z < topk, else W_alt (the shared expert); activations
-// and outputs are offset by z*x_zstride / z*y_zstride.  Plain GEMV: sel == nullptr, z = 0.
-struct RefGather {
-    const int32_t* sel;
-    int topk;
-    int64_t E;
-    int64_t wstride;
-    const uint8_t* W_alt;
-    int64_t x_zstride;
-    int64_t y_zstride;
-};
-
-template <int TYPE>
-__global__ __launch_bounds__(kRows) void k_gemv_ref(const uint8_t* __restrict__ W, int64_t N, int64_t K,
-                                                    const uint16_t* __restrict__ X, int64_t M,
-                                                    uint16_t* __restrict__ Y, float* __restrict__ Yf,
-                                                    RefGather ga) {
-    using S = Stage<TYPE>;
-    if (ga.sel) {
-        const int z = blockIdx.z;
-        if (z < ga.topk) {
-            int e = ga.sel[z];
-            e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
-            W += (int64_t)e * ga.wstride;
-        } else {
-            W = ga.W_alt;
-        }
-        X += (int64_t)z * ga.x_zstride;
-        Y += (int64_t)z * ga.y_zstride;
-        if (Yf) Yf += (int64_t)z * ga.y_zstride;
-    }
-    __shared__ uint16_t rows[kRows * S::stride];
-    __shared__ float xs[kMC][kStageW];
-    const int lane = threadIdx.x;
-    const int64_t row0 = (int64_t)blockIdx.x * kRows;
-    const int64_t m0 = (int64_t)blockIdx.y * kMC;
-    const int mcnt = (int)((M - m0) < kMC ? (M - m0) : kMC);
-    const int64_t rb = row_bytes(TYPE, K);
-    const int nfull = (int)(K / kStageW);
-    const int ktail = (int)(K - (int64_t)nfull * kStageW);   // a multiple of the type's block
-    float acc[kMC];
-#pragma unroll
-    for (int i = 0; i < kMC; ++i) acc[i] = 0.0f;
-
-    for (int st = 0; st < nfull + (ktail ? 1 : 0); ++st) {
-        const int kn = st < nfull ? kStageW : ktail;
-        __syncthreads();
-        if (kn == kStageW) {
-            for (int idx = lane; idx < kRows * S::u16; idx += kRows) {
-                const int r = idx / S::u16, c = idx - r * S::u16;
-                const int64_t n = row0 + r;
-                uint16_t v = 0;
-                if (n < N) v = *(const uint16_t*)(W + n * rb + (int64_t)st * S::bytes + 2 * c);
-                rows[r * S::stride + c] = v;
-            }
-        } else {
-            const int u16 = (int)(row_bytes(TYPE, kn) / 2);   // Q8_0: 17 words per block; F16 / BF16: kn
-            for (int idx = lane; idx < kRows * u16; idx += kRows) {
-                const int r = idx / u16, c = idx - r * u16;
-                const int64_t n = row0 + r;
-                uint16_t v = 0;
-                if (n < N) v = *(const uint16_t*)(W + n * rb + (int64_t)st * S::bytes + 2 * c);
-                rows[r * S::stride + c] = v;
-            }
-        }
-        for (int idx = lane; idx < kMC * kStageW; idx += kRows) {
-            const int mm = idx / kStageW, k = idx - mm * kStageW;
-            xs[mm][k] = mm < mcnt && k < kn ? bf16_to_f32(X[(m0 + mm) * K + (int64_t)st * kStageW + k]) : 0.0f;
-        }
-        __syncthreads();
-        if (row0 + lane < N) stage_mac<TYPE>((const uint8_t*)(rows + lane * S::stride), xs, mcnt, acc, kn);
-    }
-    const int64_t n = row0 + lane;
-    if (n < N) {
-        for (int mm = 0; mm < mcnt; ++mm) {
-            Y[(m0 + mm) * N + n] = (uint16_t)bf16_rne(acc[mm]);
-            if (Yf) Yf[(m0 + mm) * N + n] = acc[mm];
-        }
-    }
+__device__ __forceinline__ uint32_t word_of(const uint4& v, int i) {
+    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
 }
-
-// Q4_K in reference order with the weights in registers: the same operations in the same order
-// as k_gemv_ref<T_Q4_K> (so the same bits), arranged for the VALU.  Lane = output row; each
-// lane loads its row's 144-B super-block with nine 16-B loads, one block ahead of its use, and
-// the MC activation rows of the pass sit in LDS as fp32 (staged once, MC * K * 4 bytes), read
-// four at a time by every lane of the wave at one address.  Per weight: the nibble, its fp32
-// value (one byte conversion), w = D q - Mn, and for every activation row acc += x w.
-constexpr int kRefQ4LdsBytes = 128 * 1024;   // staged activations, at most
 
 // Byte B of v as fp32 in one instruction (plain C selects a bit-field extract, then the
 // conversion of byte 0).  VALU only, no hazard beyond what the hardware interlocks.
@@ -212,372 +58,408 @@ __device__ __forceinline__ float cvt_ubyte(uint32_t v) {
     return r;
 }
 
-template <int MC>
-__global__ __launch_bounds__(kRows) void k_gemv_ref_q4k(const uint8_t* __restrict__ W, int64_t N, int64_t K,
-                                                        const uint16_t* __restrict__ X, int64_t M,
-                                                        uint16_t* __restrict__ Y, float* __restrict__ Yf,
-                                                        RefGather ga) {
-    if (ga.sel) {
-        const int z = blockIdx.z;
-        if (z < ga.topk) {
-            int e = ga.sel[z];
-            e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
-            W += (int64_t)e * ga.wstride;
-        } else {
-            W = ga.W_alt;
-        }
-        X += (int64_t)z * ga.x_zstride;
-        Y += (int64_t)z * ga.y_zstride;
-        if (Yf) Yf += (int64_t)z * ga.y_zstride;
-    }
-    extern __shared__ __align__(16) float s_x[];   // [MC][K]
-    const int lane = threadIdx.x;
-    const int64_t row0 = (int64_t)blockIdx.x * kRows;
-    const int64_t m0 = (int64_t)blockIdx.y * MC;
-    const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
-    const int nsb = (int)(K / QK_K);
-    const uint32_t rb = (uint32_t)nsb * 144u;
-    const int nrows = (int)((N - row0) < kRows ? (N - row0) : kRows);
-    // this lane's row (rows past N read zeros), one block ahead
-    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W + row0 * (int64_t)rb, (uint32_t)nrows * rb);
-    const uint32_t wrow = (uint32_t)lane * rb;
-    uint4 nxt[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) nxt[i] = buf_load16(wr, wrow + 16u * (uint32_t)i);
-    // the pass's activation rows as fp32 (rows past M as zeros): chunks of 8 elements, eight
-    // chunks' loads in flight before their stores
-    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(X + m0 * K, (uint32_t)mcnt * (uint32_t)K * 2u);
-    const int nch = MC * (int)(K / 8);
-    for (int c0 = 0; c0 < nch; c0 += 8 * kRows) {
-        uint4 v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = c0 + u * kRows + lane;
-            v[u] = buf_load16(xr, c < nch ? 16u * (uint32_t)c : 0xF0000000u);   // chunk c: row c / (K / 8)
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = c0 + u * kRows + lane;
-            if (c < nch) {
-                float4* d = (float4*)(s_x + 8 * (int64_t)c);
-                d[0] = make_float4(bf16_to_f32(v[u].x & 0xFFFFu), bf16_to_f32(v[u].x >> 16),
-                                   bf16_to_f32(v[u].y & 0xFFFFu), bf16_to_f32(v[u].y >> 16));
-                d[1] = make_float4(bf16_to_f32(v[u].z & 0xFFFFu), bf16_to_f32(v[u].z >> 16),
-                                   bf16_to_f32(v[u].w & 0xFFFFu), bf16_to_f32(v[u].w >> 16));
-            }
-        }
-    }
-    __syncthreads();
-    float acc[MC];
-#pragma unroll
-    for (int i = 0; i < MC; ++i) acc[i] = 0.0f;
-    for (int b = 0; b < nsb; ++b) {
-        uint4 R[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) R[i] = nxt[i];
-        if (b + 1 < nsb) {
-#pragma unroll
-            for (int i = 0; i < 9; ++i) nxt[i] = buf_load16(wr, wrow + 144u * (uint32_t)(b + 1) + 16u * (uint32_t)i);
-        }
-        // tools/q4k_ref.py:45-60: d, dmin, the packed scales, then the 128 bytes of nibbles
-        const float d = f16_to_f32(R[0].x & 0xFFFFu);
-        const float dm = f16_to_f32(R[0].x >> 16);
-        const uint32_t s0 = R[0].y, s1 = R[0].z, s2 = R[0].w;
-        const uint32_t qd[32] = {R[1].x, R[1].y, R[1].z, R[1].w, R[2].x, R[2].y, R[2].z, R[2].w,
-                                 R[3].x, R[3].y, R[3].z, R[3].w, R[4].x, R[4].y, R[4].z, R[4].w,
-                                 R[5].x, R[5].y, R[5].z, R[5].w, R[6].x, R[6].y, R[6].z, R[6].w,
-                                 R[7].x, R[7].y, R[7].z, R[7].w, R[8].x, R[8].y, R[8].z, R[8].w};
-        const float* xb = s_x + (int64_t)b * QK_K;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            uint32_t sc, mn;
-            q4k_scale_min(j, s0, s1, s2, sc, mn);
-            const float D = d * (float)sc;
-            const float Mn = dm * (float)mn;
-            const int g = j >> 1, hi = j & 1;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {   // bytes 4c .. 4c + 3 of the 32 of sub-block pair g
-                const uint32_t v = (hi ? qd[8 * g + c] >> 4 : qd[8 * g + c]) & 0x0F0F0F0Fu;
-                const float q[4] = {cvt_ubyte<0>(v), cvt_ubyte<1>(v), cvt_ubyte<2>(v), cvt_ubyte<3>(v)};
-                const int k = 32 * j + 4 * c;
-                float4 xv[MC];
-#pragma unroll
-                for (int mm = 0; mm < MC; ++mm) xv[mm] = *(const float4*)(xb + (int64_t)mm * K + k);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float wq = D * q[e];   // q4k_weight_exact: D * q, then - Mn
-                    const float we = wq - Mn;
-#pragma unroll
-                    for (int mm = 0; mm < MC; ++mm) {
-                        const float xe = e == 0 ? xv[mm].x : e == 1 ? xv[mm].y : e == 2 ? xv[mm].z : xv[mm].w;
-                        const float p = xe * we;
-                        acc[mm] = acc[mm] + p;
-                    }
-                }
-            }
-        }
-    }
-    const int64_t n = row0 + lane;
-    if (n < N) {
-        for (int mm = 0; mm < mcnt; ++mm) {
-            Y[(m0 + mm) * N + n] = (uint16_t)bf16_rne(acc[mm]);
-            if (Yf) Yf[(m0 + mm) * N + n] = acc[mm];
-        }
-    }
-}
-
-// Q8_0, F16 and BF16 in reference order with the weights in registers, as k_gemv_ref_q4k does
-// for Q4_K: the dequantisation of k_gemv_ref's stage_mac (so the same bits).  A unit is 64
-// weights: two Q8_0 blocks (68 B, 17 dwords: needs K % 64 == 0 so every unit starts 4-B
-// aligned) or 128 B of F16 / BF16 (needs K % 64 == 0 so rows start 16-B aligned).
+// Run r of a row: weights 16 r .. 16 r + 15.  load() fetches its bytes, prepare() its scales,
+// four() dequantises weights 4 i .. 4 i + 3 exactly as the reference does.
 template <int TYPE>
-struct RegUnit {
-    static constexpr int kDw = TYPE == T_Q8_0 ? 17 : 32;   // dwords per unit
-    static constexpr int kBytes = 4 * kDw;
+struct Run;
+
+// Q4_K (tools/q4k_ref.py:45-60): half (r & 1) of sub-block j = r / 2 of super-block r / 16, the
+// low (j even) or high nibbles of one 16-B piece.  D = d * sc and D * q are exact in fp32
+// (11 + 6 + 4 bits), so f32(f32(D * q) - Mn) is one fused multiply-add; the nibbles enter it as
+// fp16 subnormals (q * 2^-24 low, 16 q * 2^-24 high), which the scale undoes exactly.
+template <>
+struct Run<T_Q4_K> {
+    uint4 h, q;
+    __device__ __forceinline__ void load(const uint8_t* row, int r) {
+        const uint8_t* b = row + (int64_t)(r >> 4) * 144;
+        h = load16_u2(b);
+        q = load16_u2(b + 16 + 32 * ((r & 15) >> 2) + 16 * (r & 1));
+    }
+    struct Scale {
+        float s, n;      // scaled D, -Mn
+        uint32_t mask;   // of two nibbles
+    };
+    __device__ __forceinline__ Scale prepare(int r) const {
+        const int j = (r & 15) >> 1, sh = 8 * (j & 3);
+        const uint32_t a0 = h.y >> sh, a1 = h.z >> sh, a2 = h.w >> sh;
+        const uint32_t hi = 0u - (uint32_t)(j >> 2);   // all ones for sub-blocks 4 .. 7
+        const uint32_t sc = (a0 & 63u & ~hi) | (((a2 & 15u) | ((a0 >> 2) & 0x30u)) & hi);
+        const uint32_t mn = (a1 & 63u & ~hi) | ((((a2 >> 4) & 15u) | ((a1 >> 2) & 0x30u)) & hi);
+        Scale s;
+        s.s = f16_to_f32(h.x & 0xFFFFu) * cvt_ubyte<0>(sc) * ((j & 1) ? 0x1p20f : 0x1p24f);
+        s.n = -(f16_to_f32(h.x >> 16) * cvt_ubyte<0>(mn));
+        s.mask = (j & 1) ? 0x00F000F0u : 0x000F000Fu;
+        return s;
+    }
+    __device__ __forceinline__ void four(const Scale& s, int i, float (&w)[4]) const {
+        typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+        const uint32_t x = word_of(q, i);
+        const h2_t a = __builtin_bit_cast(h2_t, x & s.mask), b = __builtin_bit_cast(h2_t, (x >> 8) & s.mask);
+        w[0] = __builtin_fmaf((float)a[0], s.s, s.n);
+        w[1] = __builtin_fmaf((float)b[0], s.s, s.n);
+        w[2] = __builtin_fmaf((float)a[1], s.s, s.n);
+        w[3] = __builtin_fmaf((float)b[1], s.s, s.n);
+    }
 };
 
-template <int TYPE, int MC>
-__global__ __launch_bounds__(kRows) void k_gemv_ref_reg(const uint8_t* __restrict__ W, int64_t N, int64_t K,
-                                                        const uint16_t* __restrict__ X, int64_t M,
-                                                        uint16_t* __restrict__ Y, float* __restrict__ Yf,
-                                                        RefGather ga) {
-    typedef RegUnit<TYPE> U;
-    if (ga.sel) {
-        const int z = blockIdx.z;
-        if (z < ga.topk) {
-            int e = ga.sel[z];
-            e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
-            W += (int64_t)e * ga.wstride;
-        } else {
-            W = ga.W_alt;
-        }
-        X += (int64_t)z * ga.x_zstride;
-        Y += (int64_t)z * ga.y_zstride;
-        if (Yf) Yf += (int64_t)z * ga.y_zstride;
+// Q6_K (tools/q4k_ref.py:105-124): one scale per run.
+template <>
+struct Run<T_Q6_K> {
+    uint4 ql, qh;
+    uint32_t sc, d;
+    __device__ __forceinline__ void load(const uint8_t* row, int r) {
+        const uint8_t* b = row + (int64_t)(r >> 4) * 210;
+        const int hf = (r & 15) >> 3, t = (r >> 1) & 3, o = 16 * (r & 1);
+        ql = load16_u2(b + 64 * hf + 32 * (t & 1) + o);
+        qh = load16_u2(b + 128 + 32 * hf + o);
+        sc = b[192 + (r & 15)];
+        d = *(const uint16_t*)(b + 208);
     }
-    extern __shared__ __align__(16) float s_x[];   // [MC][K]
-    const int lane = threadIdx.x;
-    const int64_t row0 = (int64_t)blockIdx.x * kRows;
-    const int64_t m0 = (int64_t)blockIdx.y * MC;
-    const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
-    const int nu = (int)(K / 64);
-    const uint32_t rb = (uint32_t)nu * (uint32_t)U::kBytes;
-    const int nrows = (int)((N - row0) < kRows ? (N - row0) : kRows);
-    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W + row0 * (int64_t)rb, (uint32_t)nrows * rb);
-    const uint32_t wrow = (uint32_t)lane * rb;
-    uint32_t nxt[U::kDw];
-    auto load_unit = [&](int u) {
-        const uint32_t o = wrow + (uint32_t)U::kBytes * (uint32_t)u;
-        if constexpr (TYPE == T_Q8_0) {
-#pragma unroll
-            for (int i = 0; i < U::kDw; ++i) nxt[i] = buf_load4(wr, o + 4u * (uint32_t)i);
-        } else {
-#pragma unroll
-            for (int i = 0; i < U::kDw / 4; ++i) {
-                const uint4 v = buf_load16(wr, o + 16u * (uint32_t)i);
-                nxt[4 * i] = v.x;
-                nxt[4 * i + 1] = v.y;
-                nxt[4 * i + 2] = v.z;
-                nxt[4 * i + 3] = v.w;
-            }
-        }
+    struct Scale {
+        float ds;
+        int sl, sh;   // shifts of the nibble and of the two high bits
     };
-    load_unit(0);
-    // the pass's activation rows as fp32 (rows past M as zeros), eight loads in flight per lane
-    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(X + m0 * K, (uint32_t)mcnt * (uint32_t)K * 2u);
-    const int nch = MC * (int)(K / 8);
-    for (int c0 = 0; c0 < nch; c0 += 8 * kRows) {
-        uint4 v[8];
+    __device__ __forceinline__ Scale prepare(int r) const {
+        const int t = (r >> 1) & 3;
+        return Scale{f16_to_f32(d) * (float)(int8_t)(uint8_t)sc, 4 * (t >> 1), 2 * t};
+    }
+    __device__ __forceinline__ void four(const Scale& s, int i, float (&w)[4]) const {
+        const uint32_t code = ((word_of(ql, i) >> s.sl) & 0x0F0F0F0Fu) | (((word_of(qh, i) >> s.sh) & 0x03030303u) << 4);
+        w[0] = s.ds * (cvt_ubyte<0>(code) - 32.0f);
+        w[1] = s.ds * (cvt_ubyte<1>(code) - 32.0f);
+        w[2] = s.ds * (cvt_ubyte<2>(code) - 32.0f);
+        w[3] = s.ds * (cvt_ubyte<3>(code) - 32.0f);
+    }
+};
+
+// Q8_0: half (r & 1) of block r / 2 (fp16 d, 32 signed bytes; tools/q4k_ref.py:126-129).
+template <>
+struct Run<T_Q8_0> {
+    uint4 q;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t* row, int r) {
+        const uint8_t* b = row + (int64_t)(r >> 1) * 34;
+        d = *(const uint16_t*)b;
+        q = load16_u2(b + 2 + 16 * (r & 1));
+    }
+    struct Scale {
+        float d;
+    };
+    __device__ __forceinline__ Scale prepare(int) const { return Scale{f16_to_f32(d)}; }
+    __device__ __forceinline__ void four(const Scale& s, int i, float (&w)[4]) const {
+        const uint32_t x = word_of(q, i);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = c0 + u * kRows + lane;
-            v[u] = buf_load16(xr, c < nch ? 16u * (uint32_t)c : 0xF0000000u);
-        }
+        for (int e = 0; e < 4; ++e) w[e] = s.d * (float)(int8_t)(uint8_t)(x >> (8 * e));
+    }
+};
+
+template <int TYPE>
+struct RunHalf {   // F16 / BF16
+    uint4 v[2];
+    __device__ __forceinline__ void load(const uint8_t* row, int r) {
+        v[0] = load16_u2(row + (int64_t)r * 32);
+        v[1] = load16_u2(row + (int64_t)r * 32 + 16);
+    }
+    struct Scale {};
+    __device__ __forceinline__ Scale prepare(int) const { return Scale{}; }
+    __device__ __forceinline__ void four(const Scale&, int i, float (&w)[4]) const {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = c0 + u * kRows + lane;
-            if (c < nch) {
-                float4* d = (float4*)(s_x + 8 * (int64_t)c);
-                d[0] = make_float4(bf16_to_f32(v[u].x & 0xFFFFu), bf16_to_f32(v[u].x >> 16),
-                                   bf16_to_f32(v[u].y & 0xFFFFu), bf16_to_f32(v[u].y >> 16));
-                d[1] = make_float4(bf16_to_f32(v[u].z & 0xFFFFu), bf16_to_f32(v[u].z >> 16),
-                                   bf16_to_f32(v[u].w & 0xFFFFu), bf16_to_f32(v[u].w >> 16));
-            }
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t hw = (word_of(v[i >> 1], 2 * (i & 1) + (e >> 1)) >> (16 * (e & 1))) & 0xFFFFu;
+            w[e] = TYPE == T_F16 ? f16_to_f32(hw) : bf16_to_f32(hw);
         }
     }
-    __syncthreads();
-    float acc[MC];
+};
+template <>
+struct Run<T_F16> : RunHalf<T_F16> {};
+template <>
+struct Run<T_BF16> : RunHalf<T_BF16> {};
+
+// ---------------------------------------------------------------- one workgroup
+// RM: row capacity of a workgroup, MC: activation rows.  RM = 32 while that leaves every CU at
+// most one workgroup (a half-empty chain wave costs nothing there), RM = 64 beyond, where the
+// workgroups of a CU share its VALU (N = 16384, K = 6144: 37 us; one row's chain alone 24 us).
+template <int MC, int RM>
+struct RefCfg {
+    static constexpr bool kMul = MC > 2;              // the chains multiply; else the producers do
+    static constexpr int NBUF = 3;
+    static constexpr int G = kMul ? 1 : MC;           // activation rows a producer lane multiplies with
+    static constexpr int RW = RM / 4;                 // rows per producer wave
+    static constexpr int RPS = 64 / RW;               // runs per stage
+    static constexpr int KS = 16 * RPS;
+    static constexpr int L = kMul ? RM : MC * RM;     // 16-B slots per four k
+    static constexpr int kXBytes = kMul ? MC * KS * 4 : 0;
+    static constexpr int kStageBytes = KS / 4 * L * 16 + kXBytes;
+    static constexpr int kChains = MC * RM <= 64 ? 1 : MC * RM / 64;
+    static constexpr int kThreads = 64 * (4 + kChains);
+    static constexpr int kLds = NBUF * kStageBytes;
+    static_assert(MC * KS <= 1024 && kLds <= 96 * 1024, "a stage must split over the producer lanes");
+};
+
+// A workgroup barrier that waits for this wave's LDS writes and nothing else: global loads for
+// later stages stay in flight.
+__device__ __forceinline__ void stage_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int TYPE, int G, bool MUL>
+struct Held {   // one stage's operands of a producer lane
+    Run<TYPE> w;
+    uint4 x[G][2];   // !MUL: the run's activations
+    uint2 xs;        // MUL: four activations to stage
+};
+
+typedef uint32_t u32x2_u2 __attribute__((ext_vector_type(2), aligned(2)));
+
+// Rows [row0, row0 + R) of W [N][K] against activation rows X [mcnt][K]; y[m * ys + row].
+// R <= RM, a multiple of 8; rows at or past N and activation rows at or past mcnt repeat the
+// last one and are not stored.
+template <int TYPE, int MC, int RM>
+__device__ __forceinline__ void ref_rows(const uint8_t* __restrict__ W, int64_t N, int64_t K,
+                                         const uint16_t* __restrict__ X, int mcnt, uint16_t* __restrict__ Y,
+                                         float* __restrict__ Yf, int64_t ys, int64_t row0, int R, uint8_t* lds) {
+    typedef RefCfg<MC, RM> C;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int S = (int)((K + C::KS - 1) / C::KS);
+    constexpr int LA = C::NBUF - 1;                       // stages between the producers and the chains
+    constexpr int kWBytes = C::kStageBytes - C::kXBytes;   // the stage's activations follow its slots
+
+    if (wave >= C::kChains) {   // producer: rows RW * pw .. of the workgroup
+        const int pw = wave - C::kChains;
+        const int un = lane / C::RW;   // run of the stage
+        const int row = pw * C::RW + lane % C::RW;
+        const int64_t n = row0 + row < N ? row0 + row : N - 1;
+        const uint8_t* wr = W + n * row_bytes(TYPE, K);
+        const uint16_t* xr[C::G];
 #pragma unroll
-    for (int i = 0; i < MC; ++i) acc[i] = 0.0f;
-    for (int u = 0; u < nu; ++u) {
-        uint32_t R[U::kDw];
-#pragma unroll
-        for (int i = 0; i < U::kDw; ++i) R[i] = nxt[i];
-        if (u + 1 < nu) load_unit(u + 1);
-        const float* xb = s_x + (int64_t)u * 64;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {   // weights 4c .. 4c + 3 of the unit
-            float w[4];
-            if constexpr (TYPE == T_Q8_0) {
-                // block c / 8: fp16 d at bytes 34 (c / 8), codes at bytes 34 (c / 8) + 2 + ..
-                const int blk = c >> 3, i0 = 4 * (c & 7);
-                const float d = f16_to_f32(blk == 0 ? (R[0] & 0xFFFFu) : (R[8] >> 16));
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int byte = 34 * blk + 2 + i0 + e;   // byte of the unit
-                    const uint32_t q = (R[byte >> 2] >> (8 * (byte & 3))) & 0xFFu;
-                    w[e] = d * (float)(int8_t)q;
-                }
+        for (int g = 0; g < C::G; ++g) xr[g] = X + (int64_t)(g < mcnt ? g : mcnt - 1) * K;
+        // MUL: the four activations of the stage this lane stages: row xm, k xk .. xk + 3
+        const int xi = pw * 64 + lane, xm = xi / (C::KS / 4), xk = 4 * (xi % (C::KS / 4));
+        const uint16_t* xsr = X + (int64_t)(xm < mcnt ? xm : mcnt - 1) * K;
+        const bool stager = C::kMul && xm < MC;
+        const bool busy = pw * C::RW < R;   // wave-uniform: a wave past the last row only stages
+        const int nr = (int)(K / 16);       // whole runs
+        // stage t's operands; runs past the last whole one repeat it (their products are not
+        // read, or come from the partial path below)
+        auto fetch = [&](Held<TYPE, C::G, C::kMul>& b, int t) {
+            int r = t * C::RPS + un;
+            r = r < nr ? r : nr - 1;
+            b.w.load(wr, r);
+            if constexpr (C::kMul) {
+                const int64_t k = (int64_t)t * C::KS + xk;
+                const u32x2_u2 v = *(const u32x2_u2*)(xsr + (k + 4 <= K ? k : K - 4));
+                b.xs = make_uint2(v.x, v.y);
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t h = (R[2 * c + (e >> 1)] >> (16 * (e & 1))) & 0xFFFFu;
-                    w[e] = TYPE == T_F16 ? f16_to_f32(h) : bf16_to_f32(h);
+                for (int g = 0; g < C::G; ++g) {
+                    b.x[g][0] = load16_u2(xr[g] + 16 * r);
+                    b.x[g][1] = load16_u2(xr[g] + 16 * r + 8);
                 }
             }
-            float4 xv[MC];
+        };
+        auto slot = [&](int buf, int k4, int g) { return lds + buf * C::kStageBytes + (k4 * C::L + g * RM + row) * 16; };
+        auto xslot = [&](int buf) { return (float*)(lds + buf * C::kStageBytes + kWBytes) + xm * C::KS + xk; };
+        // this lane's run of stage t: its products, or its weights and the activations
+        auto emit = [&](const Held<TYPE, C::G, C::kMul>& b, int t, int buf) {
+            if (C::kMul && stager)
+                *(float4*)xslot(buf) = make_float4(bf16_to_f32(b.xs.x & 0xFFFFu), __uint_as_float(b.xs.x & 0xFFFF0000u),
+                                                   bf16_to_f32(b.xs.y & 0xFFFFu), __uint_as_float(b.xs.y & 0xFFFF0000u));
+            if (!busy) return;
+            const auto sc = b.w.prepare(t * C::RPS + un);
 #pragma unroll
-            for (int mm = 0; mm < MC; ++mm) xv[mm] = *(const float4*)(xb + (int64_t)mm * K + 4 * c);
+            for (int i = 0; i < 4; ++i) {
+                float w[4];
+                b.w.four(sc, i, w);
+                if constexpr (C::kMul) {
+                    *(float4*)slot(buf, 4 * un + i, 0) = make_float4(w[0], w[1], w[2], w[3]);
+                } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                for (int mm = 0; mm < MC; ++mm) {
-                    const float xe = e == 0 ? xv[mm].x : e == 1 ? xv[mm].y : e == 2 ? xv[mm].z : xv[mm].w;
-                    const float p = xe * w[e];
-                    acc[mm] = acc[mm] + p;
-                }
-            }
-        }
-    }
-    const int64_t n = row0 + lane;
-    if (n < N) {
-        for (int mm = 0; mm < mcnt; ++mm) {
-            Y[(m0 + mm) * N + n] = (uint16_t)bf16_rne(acc[mm]);
-            if (Yf) Yf[(m0 + mm) * N + n] = acc[mm];
-        }
-    }
-}
-
-// Q6_K in reference order with the weights in registers: stage_mac's Q6_K dequantisation (so
-// the same bits).  A 210-B block starts 4-B aligned when its index is even and 2 B past a dword
-// when it is odd (K a multiple of 512, rows 4-B aligned); each lane loads the 53 dwords that
-// span its block, one block ahead, and realigns the dwords it uses by `par` (0 or 2) bytes.
-// Four weights at a time: code = nibble | 2-bit high part << 4 for four bytes in one dword,
-// then per weight (float)(code - 32) (as cvt(code) - 32, exact) times d * sc.
-__device__ __forceinline__ uint32_t q6_dword(const uint32_t (&R)[53], int o, uint32_t par) {   // bytes o .. o + 3, o % 4 == 0, o <= 204
-    return __builtin_amdgcn_alignbyte(R[(o >> 2) + 1], R[o >> 2], par);
-}
-
-template <int MC>
-__device__ __forceinline__ void q6_block_ref(const uint32_t (&R)[53], uint32_t par, const float* xb, int64_t K,
-                                             float (&acc)[MC]) {
-    const float d = f16_to_f32(par ? R[52] >> 16 : R[52] & 0xFFFFu);   // d: block bytes 208..209, the span's last dword
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            __builtin_amdgcn_sched_barrier(0);   // one run of 32 weights at a time (registers)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {   // weights 128h + 32t + 4c .. + 3
-                const uint32_t ql = q6_dword(R, 64 * h + 32 * (t & 1) + 4 * c, par);
-                const uint32_t qh = q6_dword(R, 128 + 32 * h + 4 * c, par);
-                const uint32_t code = ((t < 2 ? ql : ql >> 4) & 0x0F0F0F0Fu) | (((qh >> (2 * t)) & 0x03030303u) << 4);
-                const int si = 8 * h + 2 * t + (c >> 2);   // scale index k >> 4
-                const uint32_t sw = q6_dword(R, 192 + (si & ~3), par);
-                const float ds = d * (float)(int8_t)(uint8_t)(sw >> (8 * (si & 3)));
-                const float q[4] = {cvt_ubyte<0>(code), cvt_ubyte<1>(code), cvt_ubyte<2>(code), cvt_ubyte<3>(code)};
-                const int k = 128 * h + 32 * t + 4 * c;
-                float4 xv[MC];
-#pragma unroll
-                for (int mm = 0; mm < MC; ++mm) xv[mm] = *(const float4*)(xb + (int64_t)mm * K + k);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float w = ds * (q[e] - 32.0f);
-#pragma unroll
-                    for (int mm = 0; mm < MC; ++mm) {
-                        const float xe = e == 0 ? xv[mm].x : e == 1 ? xv[mm].y : e == 2 ? xv[mm].z : xv[mm].w;
-                        const float p = xe * w;
-                        acc[mm] = acc[mm] + p;
+                    for (int g = 0; g < C::G; ++g) {
+                        const uint4& xv = b.x[g][i >> 1];
+                        const uint32_t x0 = word_of(xv, 2 * (i & 1)), x1 = word_of(xv, 2 * (i & 1) + 1);
+                        float4 p;
+                        p.x = bf16_to_f32(x0 & 0xFFFFu) * w[0];
+                        p.y = __uint_as_float(x0 & 0xFFFF0000u) * w[1];
+                        p.z = bf16_to_f32(x1 & 0xFFFFu) * w[2];
+                        p.w = __uint_as_float(x1 & 0xFFFF0000u) * w[3];
+                        *(float4*)slot(buf, 4 * un + i, g) = p;
                     }
                 }
             }
+        };
+        // the last stage of a K that is not a multiple of 16 (F16 / BF16, any K): the last run and
+        // the activations that go with it, one element at a time
+        auto emit_partial = [&](int buf) {
+            if constexpr (TYPE == T_F16 || TYPE == T_BF16) {
+                const int kt = (int)(K % 16);
+                if (kt == 0) return;
+                const int64_t k0 = 16 * (int64_t)nr;
+                if constexpr (C::kMul) {
+                    const int64_t k = (int64_t)(S - 1) * C::KS + xk;
+                    if (stager && k < K && (k + 4 > K || nr == 0))
+                        for (int e = 0; e < 4; ++e) xslot(buf)[e] = k + e < K ? bf16_to_f32(xsr[k + e]) : 0.0f;
+                }
+                if ((S - 1) * C::RPS + un == nr) {
+                    for (int k = 0; k < kt; ++k) {
+                        const uint32_t hw = *(const uint16_t*)(wr + 2 * (k0 + k));
+                        const float w = TYPE == T_F16 ? f16_to_f32(hw) : bf16_to_f32(hw);
+#pragma unroll
+                        for (int g = 0; g < C::G; ++g)
+                            ((float*)slot(buf, 4 * un + (k >> 2), g))[k & 3] = C::kMul ? w : bf16_to_f32(xr[g][k0 + k]) * w;
+                    }
+                }
+            }
+        };
+        if (nr) {
+            // NBUF stages of loads in flight, so that every buffer index is a constant; the loop has
+            // no branch between a load and its use, so each wait is for the oldest stage's loads only
+            Held<TYPE, C::G, C::kMul> held[C::NBUF];
+#pragma unroll
+            for (int j = 0; j < C::NBUF; ++j) fetch(held[j], j);
+            int t = 0;
+            for (; t + C::NBUF < S; t += C::NBUF) {
+#pragma unroll
+                for (int j = 0; j < C::NBUF; ++j) {
+                    emit(held[j], t + j, j);
+                    fetch(held[j], t + j + C::NBUF);
+                    stage_barrier();
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < C::NBUF; ++j) {
+                if (t + j < S) {
+                    emit(held[j], t + j, j);
+                    if (t + j == S - 1) emit_partial(j);
+                    stage_barrier();
+                }
+            }
+        } else {
+            emit_partial(0);
+            stage_barrier();
         }
+#pragma unroll
+        for (int t = 0; t < LA; ++t) stage_barrier();
+        return;
+    }
+
+    // chain: lane = (activation row, row)
+    __builtin_amdgcn_s_setprio(3);
+    const int li = wave * 64 + lane;
+    const int m = li / RM, row = li % RM;
+    const bool live = row < R && m < mcnt && row0 + row < N;
+    // The chain issues a group of GR reads at once and waits once per group: a wait before every
+    // read's four adds cost 1.5 cycles per k (M = 1: 32 -> 25.5 us at 6144 x 6144).
+    constexpr int GR = 4, D = 2 * GR, kReads = C::kMul ? 2 : 1;
+    constexpr int NK4 = C::KS / 4;
+    static_assert(NK4 % D == 0, "the read ring must start every stage at q[0]");
+    const uint8_t* const base = lds + (C::kMul ? row : li) * 16;
+    const uint8_t* const xbase = lds + kWBytes + m * (C::KS * 4);
+    float acc = 0.0f;
+#pragma unroll
+    for (int t = 0; t < LA; ++t) stage_barrier();
+    float4 q[D], xq[D];
+    // reads j .. j + GR - 1 of the stage at offset oc, which runs on into the stage at offset on
+    auto read_group = [&](int j0, int oc, int on) {
+#pragma unroll
+        for (int e = 0; e < GR; ++e) {
+            const int j = j0 + e;
+            q[j % D] = *(const float4*)(base + (j < NK4 ? oc + j * C::L * 16 : on + (j - NK4) * C::L * 16));
+            if (C::kMul) xq[j % D] = *(const float4*)(xbase + (j < NK4 ? oc + j * 16 : on + (j - NK4) * 16));
+        }
+    };
+    if (live) read_group(0, 0, 0);
+    int cur = 0;
+    for (int s = 0; s < S; ++s) {
+        const int nxt = cur + 1 == C::NBUF ? 0 : cur + 1;
+        const int oc = cur * C::kStageBytes, on = nxt * C::kStageBytes;
+        if (live) {   // lanes without an output read nothing; every wave meets every barrier
+            if (s < S - 1 || K % C::KS == 0) {
+#pragma unroll
+                for (int i = 0; i < NK4; ++i) {
+                    if (i % GR == 0) {   // the group after next, then one wait for all of this group
+                        read_group(i + D - GR, oc, on);
+                        __builtin_amdgcn_s_waitcnt(0xC07F | (kReads * (D - GR)) << 8);   // lgkmcnt
+                    }
+                    float4 v = q[i % D];
+                    if constexpr (C::kMul) {
+                        const float4 x = xq[i % D];
+                        v.x = x.x * v.x;
+                        v.y = x.y * v.y;
+                        v.z = x.z * v.z;
+                        v.w = x.w * v.w;
+                    }
+                    acc = acc + v.x;
+                    acc = acc + v.y;
+                    acc = acc + v.z;
+                    acc = acc + v.w;
+                    __builtin_amdgcn_sched_barrier(0);   // the chain's order of issue is the plan
+                }
+            } else {   // the partial last stage
+                const int kn = (int)(K - (int64_t)s * C::KS);
+                for (int k = 0; k < kn; ++k) {
+                    float p = ((const float*)(base + oc + (k >> 2) * C::L * 16))[k & 3];
+                    if constexpr (C::kMul) p = ((const float*)(xbase + oc))[k] * p;
+                    acc = acc + p;
+                }
+            }
+        }
+        asm volatile("s_barrier" ::: "memory");
+        cur = nxt;
+    }
+    if (live) {
+        Y[(int64_t)m * ys + row0 + row] = (uint16_t)bf16_rne(acc);
+        if (Yf) Yf[(int64_t)m * ys + row0 + row] = acc;
+    }
 }
 
-template <int MC>
-__global__ __launch_bounds__(kRows) void k_gemv_ref_q6k(const uint8_t* __restrict__ W, int64_t N, int64_t K,
-                                                        const uint16_t* __restrict__ X, int64_t M,
-                                                        uint16_t* __restrict__ Y, float* __restrict__ Yf,
-                                                        RefGather ga) {
+// Slot gathering (MoE): blockIdx.z = slot z reads weight matrix sel[z] of the `_exps`
+// stack at W + sel[z]*wstride when z < topk, else W_alt (the shared expert); activations
+// and outputs are offset by z*x_zstride / z*y_zstride.  Slots nslots .. 2 nslots - 1 are the same
+// slots of a second stack W2 / W2_alt with outputs Y2 (gate and up in one launch: one after the
+// other they leave half the chip idle).  Plain GEMV: sel == nullptr, z = 0.
+struct RefGather {
+    const int32_t* sel;
+    int topk;
+    int nslots;
+    const uint8_t* W2;
+    const uint8_t* W2_alt;
+    uint16_t* Y2;
+    int64_t E;
+    int64_t wstride;
+    const uint8_t* W_alt;
+    int64_t x_zstride;
+    int64_t y_zstride;
+};
+
+template <int TYPE, int MC, int RM>
+__global__ __launch_bounds__((RefCfg<MC, RM>::kThreads)) void k_gemv_ref(const uint8_t* __restrict__ W, int64_t N, int64_t K,
+                                                                         const uint16_t* __restrict__ X, int64_t M,
+                                                                         uint16_t* __restrict__ Y, float* __restrict__ Yf,
+                                                                         int R, RefGather ga) {
+    extern __shared__ __align__(16) uint8_t s_ref[];
     if (ga.sel) {
-        const int z = blockIdx.z;
+        int z = blockIdx.z;
+        const uint8_t* alt = ga.W_alt;
+        if (z >= ga.nslots) {
+            z -= ga.nslots;
+            W = ga.W2;
+            alt = ga.W2_alt;
+            Y = ga.Y2;
+        }
         if (z < ga.topk) {
             int e = ga.sel[z];
             e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
             W += (int64_t)e * ga.wstride;
         } else {
-            W = ga.W_alt;
+            W = alt;
         }
         X += (int64_t)z * ga.x_zstride;
         Y += (int64_t)z * ga.y_zstride;
         if (Yf) Yf += (int64_t)z * ga.y_zstride;
     }
-    extern __shared__ __align__(16) float s_x[];   // [MC][K]
-    const int lane = threadIdx.x;
-    const int64_t row0 = (int64_t)blockIdx.x * kRows;
     const int64_t m0 = (int64_t)blockIdx.y * MC;
     const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
-    const int nsb = (int)(K / QK_K);
-    const uint32_t rb = (uint32_t)nsb * 210u;
-    const int nrows = (int)((N - row0) < kRows ? (N - row0) : kRows);
-    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W + row0 * (int64_t)rb, (uint32_t)nrows * rb);
-    const uint32_t wrow = (uint32_t)lane * rb;
-    uint32_t nxt[53];
-    auto load_block = [&](int b) {   // the dwords spanning block b (the last one may read past the row: zeros or junk)
-        const uint32_t o = wrow + ((210u * (uint32_t)b) & ~3u);
-#pragma unroll
-        for (int i = 0; i < 53; ++i) nxt[i] = buf_load4(wr, o + 4u * (uint32_t)i);
-    };
-    load_block(0);
-    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(X + m0 * K, (uint32_t)mcnt * (uint32_t)K * 2u);
-    const int nch = MC * (int)(K / 8);
-    for (int c0 = 0; c0 < nch; c0 += 8 * kRows) {
-        uint4 v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = c0 + u * kRows + lane;
-            v[u] = buf_load16(xr, c < nch ? 16u * (uint32_t)c : 0xF0000000u);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = c0 + u * kRows + lane;
-            if (c < nch) {
-                float4* d = (float4*)(s_x + 8 * (int64_t)c);
-                d[0] = make_float4(bf16_to_f32(v[u].x & 0xFFFFu), bf16_to_f32(v[u].x >> 16),
-                                   bf16_to_f32(v[u].y & 0xFFFFu), bf16_to_f32(v[u].y >> 16));
-                d[1] = make_float4(bf16_to_f32(v[u].z & 0xFFFFu), bf16_to_f32(v[u].z >> 16),
-                                   bf16_to_f32(v[u].w & 0xFFFFu), bf16_to_f32(v[u].w >> 16));
-            }
-        }
-    }
-    __syncthreads();
-    float acc[MC];
-#pragma unroll
-    for (int i = 0; i < MC; ++i) acc[i] = 0.0f;
-    for (int b = 0; b < nsb; ++b) {
-        uint32_t R[53];
-#pragma unroll
-        for (int i = 0; i < 53; ++i) R[i] = nxt[i];
-        if (b + 1 < nsb) load_block(b + 1);
-        q6_block_ref<MC>(R, (210u * (uint32_t)b) & 3u, s_x + (int64_t)b * QK_K, K, acc);
-    }
-    const int64_t n = row0 + lane;
-    if (n < N) {
-        for (int mm = 0; mm < mcnt; ++mm) {
-            Y[(m0 + mm) * N + n] = (uint16_t)bf16_rne(acc[mm]);
-            if (Yf) Yf[(m0 + mm) * N + n] = acc[mm];
-        }
-    }
+    ref_rows<TYPE, MC, RM>(W, N, K, X + m0 * K, mcnt, Y + m0 * N, Yf ? Yf + m0 * N : nullptr, N,
+                           (int64_t)blockIdx.x * R, R, s_ref);
 }
 
 // Reference order on already-dequantised fp32 weights (matmul_q4k_col on a wdeq column).
@@ -620,74 +502,52 @@ __global__ __launch_bounds__(kRows) void k_gemv_ref_f32(const float* __restrict_
     }
 }
 
+// Rows per workgroup: a multiple of 8 that spreads `rows` over the CUs, at most `cap`.
+int ref_rows_per_wg(int64_t rows, int cap) {
+    const int64_t per = 8 * (int64_t)device_cu_count();
+    const int64_t r = 8 * ((rows + per - 1) / per);
+    return (int)(r < cap ? r : cap);
+}
+
+template <int TYPE, int MC, int RM>
+hipError_t run_ref(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int64_t M, uint16_t* y, float* y_f32,
+                   int nslots, const RefGather& ga, hipStream_t st) {
+    typedef RefCfg<MC, RM> C;
+    const int R = ref_rows_per_wg(N * nslots, RM);
+    const dim3 grid((unsigned)((N + R - 1) / R), (unsigned)((M + MC - 1) / MC), (unsigned)nslots);
+    hipLaunchKernelGGL((k_gemv_ref<TYPE, MC, RM>), grid, dim3(C::kThreads), C::kLds, st, W, N, K, x, M, y, y_f32, R, ga);
+    return hipGetLastError();
+}
+
+template <int TYPE>
+hipError_t run_ref_type(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int64_t M, uint16_t* y,
+                        float* y_f32, int nslots, const RefGather& ga, hipStream_t st) {
+    if (M >= 5) return run_ref<TYPE, 8, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+    if (M >= 3) return run_ref<TYPE, 4, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+    if (M == 2) return run_ref<TYPE, 2, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+    if (N * nslots <= 32 * (int64_t)device_cu_count())
+        return run_ref<TYPE, 1, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+    return run_ref<TYPE, 1, 64>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+}
+
 }  // namespace
 
 hipError_t launch_gemv_ref_gather(int type, const void* w, int64_t N, int64_t K, const uint16_t* x, int64_t M,
                                   uint16_t* y, float* y_f32, int nslots, const int32_t* sel, int topk, int64_t E,
                                   int64_t wstride, const void* w_alt, int64_t x_zstride, int64_t y_zstride,
-                                  hipStream_t st) {
+                                  hipStream_t st, const void* w2, const void* w2_alt, uint16_t* y2) {
     const uint8_t* W = (const uint8_t*)w;
-    const RefGather ga{sel, topk, E, wstride, (const uint8_t*)w_alt, x_zstride, y_zstride};
-    // the register kernels load 16 B of activations and whole dwords / 16 B of weights at a time:
-    // the pointers they start from must be aligned for that (the ABI asks less in this mode)
-    auto al = [](const void* p, uintptr_t a) { return p == nullptr || ((uintptr_t)p & (a - 1)) == 0; };
-    const uintptr_t wa = (type == T_Q8_0 || type == T_Q6_K) ? 4 : 16;
-    const bool reg_ok = al(x, 16) && al(w, wa) && al(w_alt, wa) && (x_zstride * 2) % 16 == 0 && wstride % (int64_t)wa == 0;
-    if (reg_ok && type == T_Q4_K && K % QK_K == 0 && K * 4 <= kRefQ4LdsBytes) {
-        // the register kernel: MC activation rows per pass, as many as the staged rows allow
-        int mc = 8;
-        while (mc > 1 && (mc / 2 >= M || (int64_t)mc * K * 4 > kRefQ4LdsBytes)) mc /= 2;
-        const dim3 g4((unsigned)((N + kRows - 1) / kRows), (unsigned)((M + mc - 1) / mc), (unsigned)nslots);
-        const size_t lds = (size_t)mc * (size_t)K * 4;
-        switch (mc) {
-            case 8: hipLaunchKernelGGL(k_gemv_ref_q4k<8>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-            case 4: hipLaunchKernelGGL(k_gemv_ref_q4k<4>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-            case 2: hipLaunchKernelGGL(k_gemv_ref_q4k<2>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-            default: hipLaunchKernelGGL(k_gemv_ref_q4k<1>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-        }
-        return hipGetLastError();
-    }
-    if (reg_ok && type == T_Q6_K && K % 512 == 0 && K * 4 <= kRefQ4LdsBytes) {
-        int mc = 8;
-        while (mc > 1 && (mc / 2 >= M || (int64_t)mc * K * 4 > kRefQ4LdsBytes)) mc /= 2;
-        const dim3 g4((unsigned)((N + kRows - 1) / kRows), (unsigned)((M + mc - 1) / mc), (unsigned)nslots);
-        const size_t lds = (size_t)mc * (size_t)K * 4;
-        switch (mc) {
-            case 8: hipLaunchKernelGGL(k_gemv_ref_q6k<8>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-            case 4: hipLaunchKernelGGL(k_gemv_ref_q6k<4>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-            case 2: hipLaunchKernelGGL(k_gemv_ref_q6k<2>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-            default: hipLaunchKernelGGL(k_gemv_ref_q6k<1>, g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break;
-        }
-        return hipGetLastError();
-    }
-    if (reg_ok && (type == T_Q8_0 || type == T_F16 || type == T_BF16) && K % 64 == 0 && K * 4 <= kRefQ4LdsBytes) {
-        int mc = 8;
-        while (mc > 1 && (mc / 2 >= M || (int64_t)mc * K * 4 > kRefQ4LdsBytes)) mc /= 2;
-        const dim3 g4((unsigned)((N + kRows - 1) / kRows), (unsigned)((M + mc - 1) / mc), (unsigned)nslots);
-        const size_t lds = (size_t)mc * (size_t)K * 4;
-#define AIPU_REFREG(T)                                                                                                 \
-    switch (mc) {                                                                                                      \
-        case 8: hipLaunchKernelGGL((k_gemv_ref_reg<T, 8>), g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break; \
-        case 4: hipLaunchKernelGGL((k_gemv_ref_reg<T, 4>), g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break; \
-        case 2: hipLaunchKernelGGL((k_gemv_ref_reg<T, 2>), g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break; \
-        default: hipLaunchKernelGGL((k_gemv_ref_reg<T, 1>), g4, dim3(kRows), lds, st, W, N, K, x, M, y, y_f32, ga); break; \
-    }
-        if (type == T_Q8_0) { AIPU_REFREG(T_Q8_0) }
-        else if (type == T_F16) { AIPU_REFREG(T_F16) }
-        else { AIPU_REFREG(T_BF16) }
-#undef AIPU_REFREG
-        return hipGetLastError();
-    }
-    const dim3 grid((unsigned)((N + kRows - 1) / kRows), (unsigned)((M + kMC - 1) / kMC), (unsigned)nslots);
+    const RefGather ga{sel, topk, nslots, (const uint8_t*)w2, (const uint8_t*)w2_alt, y2, E, wstride,
+                       (const uint8_t*)w_alt, x_zstride, y_zstride};
+    if (w2) nslots *= 2;
     switch (type) {
-        case T_Q4_K: hipLaunchKernelGGL(k_gemv_ref<T_Q4_K>, grid, dim3(kRows), 0, st, W, N, K, x, M, y, y_f32, ga); break;
-        case T_Q6_K: hipLaunchKernelGGL(k_gemv_ref<T_Q6_K>, grid, dim3(kRows), 0, st, W, N, K, x, M, y, y_f32, ga); break;
-        case T_Q8_0: hipLaunchKernelGGL(k_gemv_ref<T_Q8_0>, grid, dim3(kRows), 0, st, W, N, K, x, M, y, y_f32, ga); break;
-        case T_F16: hipLaunchKernelGGL(k_gemv_ref<T_F16>, grid, dim3(kRows), 0, st, W, N, K, x, M, y, y_f32, ga); break;
-        case T_BF16: hipLaunchKernelGGL(k_gemv_ref<T_BF16>, grid, dim3(kRows), 0, st, W, N, K, x, M, y, y_f32, ga); break;
+        case T_Q4_K: return run_ref_type<T_Q4_K>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+        case T_Q6_K: return run_ref_type<T_Q6_K>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+        case T_Q8_0: return run_ref_type<T_Q8_0>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+        case T_F16: return run_ref_type<T_F16>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+        case T_BF16: return run_ref_type<T_BF16>(W, N, K, x, M, y, y_f32, nslots, ga, st);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_gemv_ref(int type, const void* w, int64_t N, int64_t K, const uint16_t* x, int64_t M,

@@ -34,11 +34,13 @@ hipError_t launch_router_bf16_logits_rows(const uint16_t* W, const uint16_t* x, 
 hipError_t launch_gemv_ref(int type, const void* w, int64_t N, int64_t K, const uint16_t* x, int64_t M,
                            uint16_t* y, float* y_f32, hipStream_t st);
 // Slot-gathered form (MoE reference path): grid z = slot; slot z < topk uses weight matrix
-// sel[z] of the stack (stride wstride bytes), slot topk the shared matrix w_alt.
+// sel[z] of the stack (stride wstride bytes), slot topk the shared matrix w_alt.  w2 / w2_alt /
+// y2 (nullable): the same slots of a second stack with its own outputs, in the same launch.
 hipError_t launch_gemv_ref_gather(int type, const void* w, int64_t N, int64_t K, const uint16_t* x, int64_t M,
                                   uint16_t* y, float* y_f32, int nslots, const int32_t* sel, int topk, int64_t E,
                                   int64_t wstride, const void* w_alt, int64_t x_zstride, int64_t y_zstride,
-                                  hipStream_t st);
+                                  hipStream_t st, const void* w2 = nullptr, const void* w2_alt = nullptr,
+                                  uint16_t* y2 = nullptr);
 hipError_t launch_gemv_ref_f32(const float* w, int64_t N, int64_t K, const float* x, int64_t M,
                                uint16_t* y, float* y_f32, hipStream_t st);
 

@@ -169,9 +169,7 @@ hipError_t launch_moe_decode(const MoeArgs& a, hipStream_t st) {
     uint16_t* ys = (uint16_t*)(ws + L.ys);
     const int64_t rbH = row_bytes(a.type, a.H), rbI = row_bytes(a.type, a.I);
     AIPU_TRY(launch_gemv_ref_gather(a.type, a.gate_exps, a.I, a.H, a.x, 1, g, nullptr, nslots, sel, a.topk, a.E,
-                                    rbH * a.I, a.sh_gate, 0, a.I, st));
-    AIPU_TRY(launch_gemv_ref_gather(a.type, a.up_exps, a.I, a.H, a.x, 1, u, nullptr, nslots, sel, a.topk, a.E,
-                                    rbH * a.I, a.sh_up, 0, a.I, st));
+                                    rbH * a.I, a.sh_gate, 0, a.I, st, a.up_exps, a.sh_up, u));
     hipLaunchKernelGGL(k_silu_mul, dim3(blocks_for(nslots * a.I)), dim3(256), 0, st, g, u, nslots * a.I, h);
     AIPU_TRY(hipGetLastError());
     AIPU_TRY(launch_gemv_ref_gather(a.type, a.down_exps, a.H, a.I, h, 1, ys, nullptr, nslots, sel, a.topk, a.E,
@@ -206,8 +204,9 @@ hipError_t launch_swiglu_expert(int type, const void* wg, const void* wu, const 
     }
     uint16_t* g = (uint16_t*)(ws + L.g);
     uint16_t* u = (uint16_t*)(ws + L.u);
-    AIPU_TRY(launch_gemv_ref(type, wg, I, H, x, 1, g, nullptr, st));
-    AIPU_TRY(launch_gemv_ref(type, wu, I, H, x, 1, u, nullptr, st));
+    // gate and up in one launch: one slot, the shared matrices (topk = 0, so the id slot is not read)
+    AIPU_TRY(launch_gemv_ref_gather(type, nullptr, I, H, x, 1, g, nullptr, 1, (const int32_t*)(ws + L.sel), 0, 1, 0, wg,
+                                    0, 0, st, wu, wu, u));
     hipLaunchKernelGGL(k_silu_mul, dim3(blocks_for(I)), dim3(256), 0, st, g, u, I, h);
     AIPU_TRY(hipGetLastError());
     return launch_gemv_ref(type, wd, H, I, h, 1, y, nullptr, st);

@@ -210,6 +210,31 @@ def test_gemv_k_not_multiple_of_256(t, N, K, M, mode):
     assert_bits_equal(h_bits(y), ye, "y")
 
 
+# Rows per workgroup are a multiple of 8 spread over the CUs (8, 16, 24 up to 32, then 64 for one
+# activation row); one or two activation rows are multiplied by the producers, more by the chains;
+# K = 15 has no whole run, K = 1553 ends 1 past a run and a four-k slot.
+SPLIT_CASES = [
+    (qo.GGML_Q4_K, 2049, 256, 1), (qo.GGML_Q6_K, 4099, 256, 2), (qo.GGML_Q8_0, 8192, 160, 1),
+    (qo.GGML_Q4_K, 8193, 512, 1), (30, 8257, 72, 1), (qo.GGML_F16, 8200, 33, 3), (qo.GGML_Q6_K, 7, 2560, 4),
+    (qo.GGML_Q8_0, 2055, 96, 8), (qo.GGML_F16, 25, 15, 8), (qo.GGML_F16, 9, 1553, 4), (30, 40, 1553, 2),
+]
+
+
+@pytest.mark.parametrize("t,N,K,M", SPLIT_CASES)
+def test_gemv_ref_row_split(t, N, K, M):
+    note(f"gemv ref split type={t} N={N} K={K} M={M}")
+    rng = np.random.default_rng(N * 31 + K + M)
+    raw = qo.random_bf16(rng, N * K).view(np.uint8) if t == 30 else qo.random_weights(rng, t, N, K)
+    x = qo.random_bf16(rng, (M, K))
+    y, yf = dev.gemv(t, d_u8(raw), N, K, d_bf16(x), mode="ref", out_f32=True)
+    if t == 30:
+        acc, ye = qo.gemv_ref(qo.bf16_bits_to_f32(raw.view(np.uint16)).reshape(N, K), qo.bf16_bits_to_f32(x))
+    else:
+        acc, ye = co.gemv_ref(t, raw, N, K, x)
+    assert_bits_equal(u32(h_f32(yf)), u32(acc), "acc")
+    assert_bits_equal(h_bits(y), ye, "y")
+
+
 def test_gemv_ref_full_north_star_shape():
     """K = N = 6144, M = 1: every output bit-exact against the C oracle."""
     note("gemv ref 6144x6144")
