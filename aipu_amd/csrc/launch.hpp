@@ -41,6 +41,9 @@ hipError_t launch_gemv_ref_gather(int type, const void* w, int64_t N, int64_t K,
                                   int64_t wstride, const void* w_alt, int64_t x_zstride, int64_t y_zstride,
                                   hipStream_t st, const void* w2 = nullptr, const void* w2_alt = nullptr,
                                   uint16_t* y2 = nullptr);
+// Tiles of any types in one launch; row m of the output starts at y + m * ys.
+hipError_t launch_gemv_ref_tiles(const aipu_tile_desc* tiles, int n_tiles, int64_t K, const uint16_t* x, int64_t M,
+                                 uint16_t* y, float* y_f32, int64_t ys, hipStream_t st);
 hipError_t launch_gemv_ref_f32(const float* w, int64_t N, int64_t K, const float* x, int64_t M,
                                uint16_t* y, float* y_f32, hipStream_t st);
 

@@ -614,6 +614,38 @@ def test_mixed_tiles_random_shapes(K, M, n_tiles):
         ok, worst = qo.tolerance_gate(wdq, xf, h_f32(yfb)[:, r0:r0 + n])
         assert ok, (t, r0, n, worst)
 
+# Ref-mode tiles share one launch, a multiple of 8 rows per workgroup: ragged tiles of all types with
+# gaps, one row up, two and four rows (producers multiply / chains multiply), five and nine (two
+# passes), and more than 32 rows per CU in all.
+@pytest.mark.parametrize("K,M,n_tiles,rows", [(512, 1, 7, 0), (768, 2, 5, 0), (256, 4, 6, 0), (512, 5, 3, 0),
+                                              (256, 9, 4, 0), (256, 1, 5, 1700)])
+def test_mixed_tiles_ref_one_launch(K, M, n_tiles, rows):
+    note(f"tiles ref K={K} M={M} tiles={n_tiles} rows={rows}")
+    rng = np.random.default_rng(K * 13 + M * 5 + n_tiles)
+    spec, N = _ragged_spec(rng, n_tiles, K)
+    if rows:   # every tile longer, the gaps kept
+        spec = [(t, r0 + i * rows, n + rows) for i, (t, r0, n) in enumerate(sorted(spec, key=lambda e: e[1]))]
+        N += rows * n_tiles
+    tw = [_tile_weights(rng, t, n, K)[0] for t, _, n in spec]
+    tiles = [(t, d_u8(r), r0, n) for (t, r0, n), r in zip(spec, tw)]
+    x = qo.random_bf16(rng, (M, K))
+    y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    yf = torch.full((M, N), -3.0, dtype=torch.float32, device="cuda")
+    dev.gemv_tiles(tiles, N, K, d_bf16(x), mode="ref", out=y, out_f32=yf)
+    gy, gf = h_bits(y), h_f32(yf)
+    covered = np.zeros(N, bool)
+    for (t, r0, n), r in zip(spec, tw):
+        if t == BF16:
+            acc, ye = qo.gemv_ref(qo.bf16_bits_to_f32(r.view(np.uint16)).reshape(n, K), qo.bf16_bits_to_f32(x))
+        else:
+            acc, ye = co.gemv_ref(t, r, n, K, x)
+        assert_bits_equal(u32(gf[:, r0:r0 + n]), u32(acc), f"tile type {t} at {r0}: acc")
+        assert_bits_equal(gy[:, r0:r0 + n], ye, f"tile type {t} at {r0}: y")
+        covered[r0:r0 + n] = True
+    assert np.all(gf[:, ~covered] == np.float32(-3.0)), "rows outside the tiles written"
+    assert np.all(gy[:, ~covered] == qo.bf16_round_bits(np.float32(7.0))), "rows outside the tiles written"
+
+
 def _tile_weights(rng, t, rows, K):
     """(raw bytes, dequantised float32[rows, K]) of a tile; BF16 tiles hold N(0, 0.05^2) bf16."""
     if t == BF16:
