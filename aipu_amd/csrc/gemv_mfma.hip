@@ -1148,7 +1148,7 @@ bool gemv_mfma_supported(int64_t N, int64_t K, int64_t M) {
 // y[M][N] (row stride ystride) = x[M][K] . W^T, in passes of at most 8 activation rows.
 // A pass goes to a multi-row kernel only if that kernel forms each row exactly as the one-row
 // launch does (two rows on the persistent one-row kernel itself, the persistent row-pair
-// kernel, k_gemvm, k_gemvs: the order of mfma_gemv.hpp,
+// kernel, k_gemvm, k_gemvs, k_gemvr: the order of mfma_gemv.hpp,
 // which the single-row kernels k_gemv1p and k_gemv1 follow); every other row runs as its own
 // one-row launch, so each row of the result is bit-identical to the one-row call on that row
 // at every shape.  `dense` swaps the persistent row-pair kernel for the dense one (rows within
@@ -1179,6 +1179,14 @@ hipError_t launch_gemv_mfma(const void* w, int64_t N, int64_t K, const uint16_t*
                 m0 += left;
                 continue;
             }
+            // the any-K kernel: beyond K = 6144, and where no kernel that holds a wave's whole part has
+            // a plan (two rows of those go to the one-row kernel above where it serves them)
+            if ((K > 6144 || !(left >= 5 ? gemvm_supported(nsb, 8) : small)) && gemv_rows_supported(N, K, left)) {
+                const hipError_t e = launch_gemv_rows(W, N, K, xm, left, ym, yfm, ystride, st);
+                if (e != hipSuccess) return e;
+                m0 += left;
+                continue;
+            }
             if (left >= 5 && gemvm_supported(nsb, 8)) {   // five to eight rows in one pass
                 const ProbPlain<8> pb{W, N, row_bytes(T_Q4_K, K), ym, yfm, ystride, left};
                 const hipError_t e = run_gemvm<8>(pb, nsb, (unsigned)((N + kTR - 1) / kTR), xm, (int)K, st);
@@ -1192,12 +1200,6 @@ hipError_t launch_gemv_mfma(const void* w, int64_t N, int64_t K, const uint16_t*
                 const hipError_t e = runs(pb, ps, (unsigned)((N + kTR - 1) / kTR), xm, (int)K, st);
                 if (e != hipSuccess) return e;
                 m0 += mr;
-                continue;
-            }
-            if (gemv_persist2_supported(N, K)) {   // no other multi-row kernel: two rows at a time
-                const hipError_t e = launch_gemv_persist2(W, N, K, xm, ym, yfm, ystride, st);
-                if (e != hipSuccess) return e;
-                m0 += 2;
                 continue;
             }
         }

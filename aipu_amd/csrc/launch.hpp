@@ -89,6 +89,12 @@ hipError_t wait_gave_up_gemv_persist(uint32_t* flag);
 hipError_t wait_gave_up_gemv_persist_m(uint32_t* flag);
 hipError_t wait_gave_up_moe_persist(uint32_t* flag);
 
+// gemv_rows.hip -- Q4_K GEMV of 2 .. 8 activation rows at any K, one weight pass (tolerance mode,
+// each row bit-identical to the single-row kernels)
+bool gemv_rows_supported(int64_t N, int64_t K, int M);
+hipError_t launch_gemv_rows(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int M, uint16_t* y, float* yf,
+                            int64_t ys, hipStream_t st);
+
 // gemv_mfma.hip -- matrix-core Q4_K GEMV (tolerance mode).  dense = false: every row of a
 // batch is bit-identical to the one-row launch on that row; dense = true allows the dense
 // multi-row kernel (rows within the tolerance of their one-row results)

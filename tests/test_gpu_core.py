@@ -360,6 +360,29 @@ def test_gemv_fast_batch_invariance(N, K, M):
     assert ok, f"batch of M={M}: fp32 accumulators {worst:.3f} of the tolerance"
 
 
+# The any-K multi-row kernel (K > 6144, or a block count without another multi-row plan): one block per
+# wave and fewer blocks than waves, an odd part per wave, a ragged tile, 2..8 rows (both MFMA sets,
+# rows past M in a set), passes of 8 + remainder, and K past the two-workgroups-per-CU LDS plan.
+ANY_K_CASES = [(17, 8448, 2), (100, 12288, 3), (16, 10240, 5), (33, 32768, 8), (40, 49152, 6), (5, 7424, 4), (640, 5632, 8),
+               (300, 2816, 3), (48, 4352, 7), (8200, 6400, 2), (70, 8192, 10)]
+
+
+@pytest.mark.parametrize("N,K,M", ANY_K_CASES)
+def test_gemv_fast_any_k_rows(N, K, M):
+    note(f"gemv fast any K N={N} K={K} M={M}")
+    rng = np.random.default_rng(17 * N + K + M)
+    raw = qo.random_q4k_blocks(rng, N * K // 256)
+    x = qo.random_bf16(rng, (M, K))
+    wd = d_u8(raw)
+    yb, yfb = _fast_rows(qo.GGML_Q4_K, wd, N, K, x, "fast")
+    for r in range(M):
+        y1, yf1 = _fast_rows(qo.GGML_Q4_K, wd, N, K, x[r:r + 1], "fast")
+        assert_bits_equal(yf1[0], yfb[r], f"row {r} of M={M}: fp32 accumulators")
+        assert_bits_equal(y1[0], yb[r], f"row {r} of M={M}: bf16 outputs")
+    ok, worst = qo.tolerance_gate(qo.dequant_q4k(raw).reshape(N, K), qo.bf16_bits_to_f32(x), yfb.view(np.float32), rel=1e-5)
+    assert ok, f"batch of M={M}: fp32 accumulators {worst:.3f} of the tolerance"
+
+
 def _random_fast_cases(n=20, seed=1202):
     """Seeded Q4_K shapes for the fast mode's kernel choice: N from one tile to many per CU, K from
     one block to 8192 (one- and two-pair persistent waves, odd block counts), M = 1..8."""
