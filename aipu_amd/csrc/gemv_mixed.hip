@@ -24,7 +24,8 @@
 //   Q8_0 (tools/q4k_ref.py:126-129): q + 128 = byte ^ 0x80 as fp16 1024 + q + 128 (0x6400 | byte);
 //        a chain of four MFMAs per 32-weight block, seeded with -1152 * sum a, ends at sum a q,
 //        then acc += d * chain;
-//   F16 / BF16 (tools/glm_model_q4k_ref.py:61-63): the weights themselves, one chain per part.
+//   F16 / BF16 (tools/glm_model_q4k_ref.py:61-63): the weights themselves, one chain per part (F16)
+//        or per block (BF16).
 // bf16 operands (Q4_K, Q6_K, BF16) take the activations as they are.  fp16 operands (Q8_0, F16)
 // take them scaled by 2^-e, e per activation row and wave, chosen so that the largest magnitude
 // of the wave's part lies in [2^14, 2^15): every bf16 value down to 2^-31 of that maximum
@@ -516,6 +517,7 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
     } else {
         // 16 rows x 1 block: two chains (MFMAs 0..3 and 4..7 of every block) over the whole part
         f32x4_t D0 = {0.f, 0.f, 0.f, 0.f}, D1 = {0.f, 0.f, 0.f, 0.f};
+        float acc1[MR] = {}, p0[MR] = {}, p1[MR] = {};
         for (int gi = 0; gi < NG; ++gi) {
             __builtin_amdgcn_s_waitcnt(kWaitVm0);
             const uint8_t* p = wW + rrow + 128 * g;
@@ -536,13 +538,25 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
                     D0 = mfma_h(A[s], b0, D0);
                     D1 = mfma_h(A[4 + s], b1, D1);
                 } else {
-                    D0 = mfma(A[s], b0, D0);
-                    D1 = mfma(A[4 + s], b1, D1);
+                    D0 = mfma(A[s], b0, s ? D0 : f32x4_t{0.f, 0.f, 0.f, 0.f});
+                    D1 = mfma(A[4 + s], b1, s ? D1 : f32x4_t{0.f, 0.f, 0.f, 0.f});
+                }
+            }
+            if constexpr (TYPE == T_BF16) {
+                // BF16 chains end with the block and alternate between two sums each: chains over a
+                // whole part were 20 % further from the 64-bit sums than the streaming kernel's FMAs
+#pragma unroll
+                for (int m = 0; m < MR; ++m) {
+                    const float n0 = p0[m] + D0[m], n1 = p1[m] + D1[m];
+                    p0[m] = acc[m];
+                    p1[m] = acc1[m];
+                    acc[m] = n0;
+                    acc1[m] = n1;
                 }
             }
         }
 #pragma unroll
-        for (int m = 0; m < MR; ++m) acc[m] = D0[m] + D1[m];
+        for (int m = 0; m < MR; ++m) acc[m] = TYPE == T_F16 ? D0[m] + D1[m] : (acc[m] + p0[m]) + (acc1[m] + p1[m]);
     }
     // a wave with no blocks still has its (all-zero) first group in flight
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
@@ -564,6 +578,16 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
 #pragma unroll
         for (int k = 0; k < kMixW; ++k) v += red[(m * kMixW + k) * kTR + rr];
         const int64_t row = T.row0 + r0 + rr;
+        if constexpr (TYPE == T_BF16) {
+            // an infinite weight meets the zeros of the other K-groups' operands: a NaN is formed again
+            // without them, so that only a NaN of the product itself stays one
+            if (v != v) {
+                const uint16_t* wv = (const uint16_t*)(T.w + (int64_t)(r0 + rr) * rb);
+                v = 0.f;
+                for (int k = 0; k < K; ++k)
+                    v = __builtin_fmaf(bf16_to_f32(X[(int64_t)m * K + k]), bf16_to_f32(wv[k]), v);
+            }
+        }
         Y[(int64_t)m * ys + row] = (uint16_t)bf16_rne(v);
         if (Yf) Yf[(int64_t)m * ys + row] = v;
     }

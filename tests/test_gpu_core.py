@@ -426,6 +426,49 @@ def test_gemv_fast_batch_invariance_bf16(N, K, M):
         assert_bits_equal(y1[0], yb[r], f"bf16 row {r} of M={M}: bf16 outputs")
 
 
+# bf16 weights take the matrix cores up to K = 2560, and up to K = 6144 from 2048 rows on, else the
+# streaming kernel: both sides of each line, ragged row groups, batches in passes of four.
+@pytest.mark.parametrize("N,K,M", [(33, 2560, 1), (2047, 2816, 2), (2049, 2816, 3), (2050, 6144, 5), (70, 6400, 4), (15, 256, 8)])
+def test_gemv_fast_bf16_dispatch(N, K, M):
+    note(f"gemv fast bf16 dispatch N={N} K={K} M={M}")
+    rng = np.random.default_rng(19 * N + K + M)
+    wb = qo.random_bf16(rng, (N, K), scale=0.05)
+    x = qo.random_bf16(rng, (M, K))
+    wd = d_u8(wb.view(np.uint8).reshape(-1))
+    yb, yfb = _fast_rows(go.BF16_TYPE, wd, N, K, x, "fast")
+    ok, worst = qo.tolerance_gate(qo.bf16_bits_to_f32(wb), qo.bf16_bits_to_f32(x), yfb.view(np.float32))
+    assert ok, worst
+    for r in range(M):
+        y1, yf1 = _fast_rows(go.BF16_TYPE, wd, N, K, x[r:r + 1], "fast")
+        assert_bits_equal(yf1[0], yfb[r], f"row {r}: fp32 accumulators")
+        assert_bits_equal(y1[0], yb[r], f"row {r}: bf16 outputs")
+
+
+@pytest.mark.parametrize("N,K", [(40, 512), (40, 4096)])
+def test_gemv_fast_bf16_infinities(N, K):
+    """An infinite weight or activation gives the infinity of the plain sum, a NaN or inf - inf a NaN,
+    and every other output is as without them (matrix-core and streaming kernels)."""
+    note(f"gemv fast bf16 infinities N={N} K={K}")
+    rng = np.random.default_rng(N + K)
+    w = qo.bf16_bits_to_f32(qo.random_bf16(rng, (N, K), scale=0.05))
+    x = qo.bf16_bits_to_f32(qo.random_bf16(rng, (2, K)))
+    x[x == 0] = 1.0
+    w[3, 5], w[4, K - 1], w[5, 70] = np.inf, -np.inf, np.nan
+    w[6, 1], w[6, 300] = np.inf * np.sign(x[0, 1]), -np.inf * np.sign(x[0, 300])   # inf - inf in row 0
+    bits = (w.view(np.uint32) >> 16).astype(np.uint16)
+    xb = (x.view(np.uint32) >> 16).astype(np.uint16)
+    _, yf = _fast_rows(go.BF16_TYPE, d_u8(bits.reshape(-1).view(np.uint8)), N, K, xb, "fast")
+    got = yf.view(np.float32)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32)) and np.array_equal(np.isinf(got), inf)
+    fin = np.isfinite(want[0])
+    ok, worst = qo.tolerance_gate(w[fin], x[:1], got[:1, fin])
+    assert ok, worst
+
+
 # AIPU_MODE_FAST_DENSE: Q4_K batches of 2..8 rows at K = 2048/4096/6144 run the dense
 # multi-row kernel.  A row agrees with its one-row call within the fast-mode tolerance (fp32
 # gate, bf16 within 1 ulp where well conditioned), and its bits depend neither on the other
