@@ -513,6 +513,147 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 
     }
 }
 
+// ---------------------------------------------------------------- small grids: K split over the waves
+// With fewer 128 x 256 tiles than CUs, k_prefill_gemm leaves CUs idle and takes a whole walk over K
+// (112 us at K = 6144) whatever M and N are.  Here a workgroup owns 16 MS x 32 outputs and its eight
+// waves an eighth of the super-blocks each: eight times the workgroups along N, an eighth of the
+// walk.  A wave reads its activation operands straight from the staged chunks (nothing of them is
+// shared in the workgroup, every CU of an XCD reads the same chunks from its L2) and its weights
+// straight from the blocks; per super-block the arithmetic is k_prefill_gemm's.  The waves' sums meet
+// in LDS and are added in wave order.  Bound by the latency of a wave's serial steps (operand reads
+// from L2, weight rows 144 B at a time), with one or two workgroups per CU.
+constexpr int kSplitW = 8;
+constexpr int kRedStride = 36;   // floats per output row of a wave's sums: 16-column writes of four row groups on 64 banks
+
+template <int MS, int R>
+__global__ __launch_bounds__(kSplitW * 64) __attribute__((amdgpu_waves_per_eu(R == 3 ? 2 : 4))) void k_prefill_split(
+    const uint8_t* __restrict__ W, int64_t N, int nsb, const uint8_t* __restrict__ ws, const int32_t* __restrict__ rexp,
+    int M, uint16_t* __restrict__ Y, float* __restrict__ Yf, int ntiles) {
+    extern __shared__ __align__(16) float s_red[];   // [wave][16 MS][kRedStride]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    const int mt = blockIdx.x / ntiles, nt = blockIdx.x - mt * ntiles;   // the tiles of one mt run together: one set of chunks
+    const int64_t rb = (int64_t)nsb * 144;
+    const int64_t row0 = (int64_t)nt * 32;
+    const int nvalid = (int)(N - row0 < 32 ? N - row0 : 32);
+    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W + row0 * rb, (uint32_t)(nvalid * rb));
+    const int i0 = mt * MS % kMT;
+    const uint8_t* const chunks = ws + (int64_t)(mt * MS / kMT) * nsb * kChunk + i0 * 1024 + lane * 16;
+    const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f4_t acc[MS][2];
+#pragma unroll
+    for (int i = 0; i < MS; ++i) acc[i][0] = acc[i][1] = zero;
+    const CodeMask cm = code_mask();
+    const int b0 = w * nsb / kSplitW, b1 = (w + 1) * nsb / kSplitW;
+    struct Wt {
+        uint4 h[2], q[2][2];   // [subtile], [half][subtile]
+    };
+    auto load_w = [&](int b) {
+        Wt t;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t o = (uint32_t)(16 * j + n) * (uint32_t)rb + 144u * (uint32_t)b;
+            t.h[j] = buf_load16(wr, o);
+            t.q[0][j] = buf_load16(wr, o + 16u + 16u * (uint32_t)g);
+            t.q[1][j] = buf_load16(wr, o + 80u + 16u * (uint32_t)g);
+        }
+        return t;
+    };
+    auto load_a = [&](int b, int t, h8_t(&A)[MS]) {   // t = 8: the sum operands
+        const uint8_t* p = chunks + (int64_t)b * kChunk + t * (kMT * 1024);
+#pragma unroll
+        for (int i = 0; i < MS; ++i) A[i] = __builtin_bit_cast(h8_t, *(const uint4*)(p + i * 1024));
+    };
+    if (b0 < b1) {
+        Wt cur = load_w(b0);
+        // a ring of R steps of operands (nine steps per super-block: eight MFMAs and the sums), R - 1
+        // in flight; R = 3 divides nine, R = 2 starts every super-block at A[0] again
+        h8_t A[R][MS];
+        auto step = [&](int b, int t, h8_t(&dst)[MS]) {   // step t of super-block b, t up to 8 + R
+            load_a(t < 9 ? b : b + 1 < b1 ? b + 1 : b, t < 9 ? t : t - 9, dst);
+        };
+#pragma unroll
+        for (int t = 0; t < R - 1; ++t) step(b0, t, A[t]);
+        for (int b = b0; b < b1; ++b) {
+            const int bn = b + 1 < b1 ? b + 1 : b;
+            const Wt nxt = load_w(bn);
+            f4_t D1[MS][2];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                step(b, t + R - 1, A[(t + R - 1) % R]);
+                h8_t B[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    B[j] = b_operand(dword_of(cur.q[t >> 2][j], t & 3), chunk_consts(cur.h[j], g, t >> 2), cm);
+#pragma unroll
+                for (int i = 0; i < MS; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        D1[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t % R][i], B[j], t == 0 ? zero : D1[i][j], 0, 0, 0);
+            }
+            if (R == 3) step(b, 10, A[1]);
+            // the min term and the epilogue of block_epilogue
+            float d[2], dm[2];
+            u32x4_t bm[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                d[j] = f16_to_f32(cur.h[j].x);
+                dm[j] = f16_to_f32(cur.h[j].x >> 16);
+                bm[j] = min_operand(cur.h[j], g);
+            }
+            f4_t D2[MS][2];
+#pragma unroll
+            for (int i = 0; i < MS; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    D2[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8_t, A[8 % R][i]),
+                                                                       __builtin_bit_cast(bf8_t, bm[j]), zero, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[i][j][r] = __builtin_fmaf(d[j], D1[i][j][r], acc[i][j][r]);
+                        acc[i][j][r] = __builtin_fmaf(-dm[j], D2[i][j][r], acc[i][j][r]);
+                    }
+                }
+            if (R == 2) load_a(bn, 0, A[0]);
+            cur = nxt;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MS; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s_red[(w * 16 * MS + 16 * i + 4 * g + r) * kRedStride + 16 * j + n] = acc[i][j][r];
+    __syncthreads();
+    const int col = tid & 31;
+#pragma unroll
+    for (int o = tid >> 5; o < 16 * MS; o += kSplitW * 2) {
+        const int64_t m = (int64_t)mt * (16 * MS) + o;
+        if (m < M && col < nvalid) {
+            float v = s_red[o * kRedStride + col];
+#pragma unroll
+            for (int k = 1; k < kSplitW; ++k) v += s_red[(k * 16 * MS + o) * kRedStride + col];
+            v = __builtin_ldexpf(v, rexp[m]);
+            Y[m * N + row0 + col] = (uint16_t)bf16_rne(v);
+            if (Yf) Yf[m * N + row0 + col] = v;
+        }
+    }
+}
+
+// 16-row subtiles of the split kernel's tile for this shape, 0 where the 128 x 256 kernel is faster.
+// The smallest tile (the shortest walk per super-block) that leaves every
+// CU at most one workgroup, and no larger than M needs; up to six workgroups per CU in all.  Measured
+// at K = 6144, 128 x 256 kernel > split (M x N): 16 x 6144 108 > 18 us, 64 x 2048 112 > 19, 64 x 6144
+// 112 > 25, 100 x 6144 117 > 36, 256 x 6144 118 > 57, 512 x 6144 119 > 95, 128 x 16384 121 > 68;
+// beyond, 256 x 16384 123 and 123, 512 x 16384 133 against 237.
+int split_tile(int64_t M, int64_t N) {
+    const int64_t nt = (N + 31) / 32, cus = device_cu_count();
+    const auto wgs = [&](int ms) { return (M + 16 * ms - 1) / (16 * ms) * nt; };
+    const int ms = M <= 16 || wgs(1) <= cus ? 1 : M <= 32 || wgs(2) <= cus ? 2 : 4;
+    return wgs(ms) <= 6 * cus ? ms : 0;
+}
+
 int64_t mpad(int64_t M) { return (M + kBM - 1) / kBM * kBM; }
 
 }  // namespace
@@ -532,9 +673,12 @@ hipError_t launch_gemm_prefill(int type, const void* w, int64_t N, int64_t K, co
     if ((int64_t)mtiles * ntiles > 0x7FFFFFFF || (int64_t)64 * nsb * 144 >= (1LL << 32)) return hipErrorInvalidValue;
     uint8_t* chunks = (uint8_t*)ws;
     int32_t* rexp = (int32_t*)(chunks + (int64_t)mtiles * nsb * kChunk);
+    const int ms = split_tile(M, N);   // 16-row subtiles of the split kernel's tile, 0: the 128 x 256 kernel
+    // rows staged: what the GEMM reads
+    const int64_t Ms = ms ? (M + 16 * ms - 1) / (16 * ms) * (16 * ms) : Mp;
     if (K <= kStageMaxK) {
         const int items = kStageRows * 8 * nsb;
-        const dim3 grid((unsigned)(Mp / kStageRows));
+        const dim3 grid((unsigned)(Ms / kStageRows));
         const auto threads = [&](int ipt) { return dim3((unsigned)((items + 64 * ipt - 1) / (64 * ipt) * 64)); };
         if (items <= 1024)
             hipLaunchKernelGGL(k_prefill_stage<1>, grid, threads(1), 0, st, x, K, (int)M, rexp, chunks, nsb);
@@ -547,6 +691,20 @@ hipError_t launch_gemm_prefill(int type, const void* w, int64_t N, int64_t K, co
         hipLaunchKernelGGL(k_prefill_rowexp, dim3((unsigned)Mp), dim3(256), 0, st, x, K, (int)M, rexp);
         hipLaunchKernelGGL(k_prefill_pack, dim3((unsigned)nsb, (unsigned)mtiles, kBM * 8 / 256), dim3(256), 0, st, x, K,
                            (int)M, rexp, chunks, nsb);
+    }
+    if (ms) {
+        const int64_t nt = (N + 31) / 32;
+        const dim3 grid((unsigned)(Ms / (16 * ms) * nt));
+        const size_t lds = (size_t)kSplitW * 16 * ms * kRedStride * 4;
+        const auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kSplitW * 64), lds, st, (const uint8_t*)w, N, nsb, chunks, rexp, (int)M, y,
+                               y_f32, (int)nt);
+        };
+        if (ms == 1) go(k_prefill_split<1, 2>);
+        else if (ms == 2) go(k_prefill_split<2, 2>);
+        else if (grid.x <= (unsigned)device_cu_count()) go(k_prefill_split<4, 3>);
+        else go(k_prefill_split<4, 2>);
+        return hipGetLastError();
     }
     hipLaunchKernelGGL(k_prefill_gemm, dim3((unsigned)(mtiles * ntiles)), dim3(kWaves * 64), 0, st,
                        (const uint8_t*)w, N, nsb, chunks, rexp, (int)M, y, y_f32, mtiles, (int)ntiles);

@@ -53,6 +53,22 @@ def test_prefill_tolerance_shapes(M, N, K):
     _check(raw, N, K, x, y, yf, f"M={M} N={N} K={K}")
 
 
+# The split kernel's tiles (16, 32 and 64 rows; 64 with one and with more workgroups per CU) at ragged M
+# and N, fewer super-blocks than waves and uneven parts; and the 128 x 256 kernel ragged on both sides.
+SPLIT_CASES = [(16, 6001, 512), (1, 33, 256), (17, 4200, 512), (40, 4100, 256), (33, 8200, 512), (32, 16400, 256),
+               (300, 40, 2304), (5, 24, 1792), (130, 16400, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", SPLIT_CASES)
+def test_prefill_split_tiles(M, N, K):
+    note(f"prefill split M={M} N={N} K={K}")
+    rng = np.random.default_rng(M * 11 + N * 5 + K)
+    raw = qo.random_q4k_blocks(rng, N * K // 256)
+    x = qo.random_bf16(rng, (M, K))
+    y, yf = _prefill(raw, N, K, x)
+    _check(raw, N, K, x, y, yf, f"M={M} N={N} K={K}")
+
+
 def test_prefill_activation_range():
     """Rows at very different magnitudes (2^-120 .. 2^100), an all-zero row, a row mixing huge
     and tiny values, negative zeros: the per-row power-of-two scaling keeps them exact."""
