@@ -125,8 +125,9 @@ def check(rc, what):
 
 def call(name, *args):
     """Call a status-returning entry point; raise AipuError on a non-zero status."""
-    rc = getattr(lib(), name)(*args)
-    check(rc, name)
+    rc = getattr(_lib or lib(), name)(*args)
+    if rc:
+        check(rc, name)
     return rc
 
 

@@ -7,6 +7,7 @@ uint8 tensors holding ggml row blocks ``[N][K/QK][bytes]``; activations and outp
 """
 from __future__ import annotations
 
+import array
 import ctypes
 
 import torch
@@ -38,12 +39,20 @@ def _gemv_mode(mode):
     return _mode(mode)
 
 
+# A small call is bound by this module's own time (512 x 2048 GEMV: 8.1 us a call, the kernel 2.9), so
+# pointers and streams go to ctypes as plain integers and the stream comes without a Stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream of t's device as an integer handle."""
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _need_cuda(*ts):
@@ -52,9 +61,12 @@ def _need_cuda(*ts):
             raise ValueError("aipu_amd device API needs tensors on a GPU device")
 
 
+_BF16_TYPES = frozenset((torch.bfloat16, torch.int16, torch.uint16))
+
+
 def _bf16(t):
-    if t.dtype in (torch.bfloat16, torch.int16, torch.uint16):
-        return t.contiguous()
+    if t.dtype in _BF16_TYPES:
+        return t if t.is_contiguous() else t.contiguous()
     raise TypeError(f"activations must be bfloat16 (or 16-bit bf16 patterns), got {t.dtype}")
 
 
@@ -124,10 +136,12 @@ def gemv_tiles(tiles, N, K, x, mode="fast", out=None, out_f32=False):
     if x.dim() == 1:
         x = x[None]
     M = x.shape[0]
-    arr = (TileDesc * len(tiles))()
-    for i, (t, w, r0, nr) in enumerate(tiles):
-        _need_cuda(w)
-        arr[i] = TileDesc(int(t), 0, w.data_ptr(), int(r0), int(nr))
+    flat = []   # a descriptor is four 64-bit words: type (and the reserved zero above it), w, row0, nrows
+    for t, w, r0, nr in tiles:
+        if not w.is_cuda:
+            _need_cuda(w)
+        flat += (int(t) & 0xFFFFFFFF, w.data_ptr(), int(r0), int(nr))
+    arr = (TileDesc * len(tiles)).from_buffer(array.array("q", flat))
     y = out if out is not None else torch.zeros((M, N), dtype=torch.bfloat16, device=x.device)
     if isinstance(out_f32, torch.Tensor):   # caller-provided fp32 output (rows outside tiles kept)
         yf = out_f32
