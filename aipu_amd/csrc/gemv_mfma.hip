@@ -744,6 +744,18 @@ __global__ __launch_bounds__(kMaxW * 64) void k_gemvm(Prob pb, const uint16_t* _
 // CU's LDS, so two workgroups share a CU as in the M = 1 kernel.
 constexpr int kSmallMaxRows = 4;
 
+// A problem with kPairs has its own activation rows per workgroup: begin(wg) reads them (false: past
+// the grid's live end), rows() is their number, xrow(m) row m's place in act()'s xrows() rows.  Any
+// other problem's workgroups all take rows 0 .. M - 1.
+template <class Prob, class = void>
+struct HasPairs {
+    static constexpr bool v = false;
+};
+template <class Prob>
+struct HasPairs<Prob, std::void_t<decltype(Prob::kPairs)>> {
+    static constexpr bool v = Prob::kPairs;
+};
+
 template <int GS, int NW, int MR, class Prob>   // MR = 2: rows 0, 1 only; MR = 4: up to four rows
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_gemvs(
     Prob pb, const uint16_t* __restrict__ X0, int K) {
@@ -761,9 +773,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: the copies take a scalar LDS base
     const int nsb = K / QK_K;
     const int wg = blockIdx.x;
-    if (!pb.active(wg)) return;   // workgroup-uniform: past a data-dependent grid end
+    constexpr bool kPairs = HasPairs<Prob>::v;
+    int rows = 0, xrows = 0, xr0 = 0, xr1 = 0;   // rows: 1 .. MR
+    if constexpr (kPairs) {
+        if (!pb.begin(wg)) return;   // workgroup-uniform: past a data-dependent grid end
+        rows = pb.rows();
+        xrows = pb.xrows();
+        xr0 = pb.xrow(0);
+        xr1 = pb.xrow(1);
+    } else {
+        if (!pb.active(wg)) return;
+        rows = xrows = pb.M;
+    }
     const uint16_t* __restrict__ X = pb.act(wg, X0);
-    const int rows = pb.M;   // 1 .. MR
     uint8_t* wA = s_act + (uint32_t)w * kPair;
     uint8_t* wW = s_w + (uint32_t)w * Dma<GS>::kBytes;
     const TileRef tr = pb.tile(wg, 0);
@@ -771,13 +793,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     const int64_t rb = (int64_t)nsb * 144;
 
     // Activation pieces of rows r0, r0 + 1 (rows >= M read as zero).
-    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(X, (uint32_t)((int64_t)pb.M * K * 2));
+    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(X, (uint32_t)((int64_t)xrows * K * 2));
     auto load_pair = [&](int r0, uint4(&xv)[XI]) {
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             const int q = lane + 64 * i;
             const int m = q >= XP ? 1 : 0, p = q - m * XP;
-            const uint32_t off = q < 2 * XP ? 2u * (uint32_t)((r0 + m) * K + kb0 * QK_K) + 16u * (uint32_t)p : kOOB;
+            const int xm = kPairs ? (m ? xr1 : xr0) : r0 + m;
+            const bool in = q < 2 * XP && (!kPairs || m < rows);
+            const uint32_t off = in ? 2u * (uint32_t)(xm * K + kb0 * QK_K) + 16u * (uint32_t)p : kOOB;
             xv[i] = buf_load16(xr, off);
         }
     };
@@ -1360,33 +1384,59 @@ struct ProbUDown {
     }
 };
 
-// The down leg of a two-row pass: workgroup (u * htilesT + it) computes tiles NT it .. NT it +
-// NT - 1 of slot u (each copied while the one before computes), each exactly as ProbUDown<2>
-// would.
+// A slot of one or two activation rows (moe_batched.hip): expert (-1: the shared one) and
+// row | row << 4 | two << 8.  The slot and the live count are read together: one after the other
+// put a second memory round trip before every workgroup's first weight copy (two rows, 256
+// experts, 1792 x 768: 33.0 -> 29.5 us a step).
+struct Slot {
+    int e, rows;
+    __device__ __forceinline__ bool read(const int2* slots, const int32_t* nslots, int u) {
+        const int2 s = slots[u];
+        int live = __builtin_amdgcn_readfirstlane(*nslots);
+        e = __builtin_amdgcn_readfirstlane(s.x);
+        rows = __builtin_amdgcn_readfirstlane(s.y);
+        asm volatile("" : "+s"(e), "+s"(rows), "+s"(live));   // all three loads before the branch on one
+        return u < live;
+    }
+};
+
+// The down leg on slots of up to two rows: workgroup (u * htilesT + it) computes tiles NT it ..
+// NT it + NT - 1 of slot u (each copied while the one before computes), each exactly as
+// ProbUDown<2> would.  h [slot][S][I], y [slot][S][H].  Without `slots`, slot u is the union's
+// expert uidx[u] with S rows.
 template <int NT>
 struct ProbUDownT {
     const uint8_t *D, *shD;
-    const int32_t* uidx;
-    const int32_t* nslots;
-    int htilesT, M;
+    const int2* slots;
+    const int32_t *uidx, *nslots;
+    int htilesT, S;
     int64_t rb, ebytes, I, H;
     const uint16_t* h;
     uint16_t* y;
+    Slot s;
     static constexpr uint32_t kPolicy = kNT;
     static constexpr int kTiles = NT;
-    __device__ bool active(int wg) const { return wg / htilesT < *nslots; }
-    __device__ const uint16_t* act(int wg, const uint16_t*) const { return h + (int64_t)(wg / htilesT) * M * I; }
+    static constexpr bool kPairs = true;
+    __device__ bool begin(int wg) {
+        const int u = wg / htilesT;
+        if (slots) return s.read(slots, nslots, u);
+        if (u >= *nslots) return false;
+        s.e = __builtin_amdgcn_readfirstlane(uidx[u]);
+        s.rows = 1 << 4 | (S - 1) << 8;
+        return true;
+    }
+    __device__ int rows() const { return 1 + (s.rows >> 8); }
+    __device__ int xrows() const { return rows(); }
+    __device__ int xrow(int m) const { return m; }
+    __device__ const uint16_t* act(int wg, const uint16_t*) const { return h + (int64_t)(wg / htilesT) * S * I; }
     __device__ TileRef tile(int wg, int part) const {
-        const int u = wg / htilesT, it = NT * (wg % htilesT) + part;
-        const int e = __builtin_amdgcn_readfirstlane(uidx[u]);
-        const uint8_t* base = e < 0 ? shD : D + (int64_t)e * ebytes;
+        const int it = NT * (wg % htilesT) + part;
+        const uint8_t* base = s.e < 0 ? shD : D + (int64_t)s.e * ebytes;
         const int64_t nv = H - (int64_t)it * kTR;   // a tile past H reads as zero
         return TileRef{base + (nv > 0 ? (int64_t)it * kTR * rb : 0), (int)(nv <= 0 ? 0 : nv < kTR ? nv : kTR), 0};
     }
-    __device__ void store_tiles(int wg, int n, int r, const float (&v)[NT]) const {
-        if (r >= M) return;
-        const int u = wg / htilesT;
-        uint16_t* yr = y + ((int64_t)u * M + r) * H;
+    __device__ void store_tiles(int wg, int n, int r, const float (&v)[NT]) const {   // r < rows()
+        uint16_t* yr = y + ((int64_t)(wg / htilesT) * S + r) * H;
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
             const int64_t d = (int64_t)(NT * (wg % htilesT) + k) * kTR + n;
@@ -1396,33 +1446,35 @@ struct ProbUDownT {
 };
 constexpr int kDownTiles = 4;
 
-// Gate/up with the SwiGLU fused, for the small-batch kernel: workgroup (u * itiles + it)
-// computes rows it*16.. of both the gate and the up projection of slot u (two tiles, the
-// second copied while the first computes) and writes h[u][m][i] = bf16(silu(g) * u) -- the
-// same rounding steps as the separate pass.
+// Gate/up with the SwiGLU fused on such slots: workgroup (u * itiles + it) computes rows it*16..
+// of both the gate and the up projection of slot u (two tiles, the second copied while the first
+// computes) and writes h[u][m][i] = bf16(silu(g) * u) -- the same rounding steps as the separate
+// pass.  x [M][H].
 struct ProbUGateUpH {
     const uint8_t *G, *U, *shG, *shU;
-    const int32_t* uidx;
+    const int2* slots;
     const int32_t* nslots;
     int itiles, M;
     int64_t rb, ebytes, I;
     uint16_t* h;
+    Slot s;
     static constexpr uint32_t kPolicy = kNT;   // streaming (default caching measured slower here)
     static constexpr int kTiles = 2;
-    __device__ bool active(int wg) const { return wg / itiles < *nslots; }
+    static constexpr bool kPairs = true;
+    __device__ bool begin(int wg) { return s.read(slots, nslots, wg / itiles); }
+    __device__ int rows() const { return 1 + (s.rows >> 8); }
+    __device__ int xrows() const { return M; }
+    __device__ int xrow(int m) const { return (s.rows >> (4 * m)) & 15; }
     __device__ const uint16_t* act(int, const uint16_t* X) const { return X; }
     __device__ TileRef tile(int wg, int part) const {
-        const int u = wg / itiles, it = wg % itiles;
-        const int e = __builtin_amdgcn_readfirstlane(uidx[u]);
-        const uint8_t* base = e < 0 ? (part ? shU : shG) : (part ? U : G) + (int64_t)e * ebytes;
+        const int it = wg % itiles;
+        const uint8_t* base = s.e < 0 ? (part ? shU : shG) : (part ? U : G) + (int64_t)s.e * ebytes;
         return TileRef{base + (int64_t)it * kTR * rb, kTR, 0};
     }
-    __device__ void store_tiles(int wg, int n, int r, const float (&v)[2]) const {
-        if (r >= M) return;
-        const float g = v[0];
+    __device__ void store_tiles(int wg, int n, int r, const float (&v)[2]) const {   // r < rows()
         const int u = wg / itiles, it = wg % itiles;
-        const uint32_t gb = bf16_rne(g), ub = bf16_rne(v[1]);
-        h[((int64_t)u * M + r) * I + (int64_t)it * kTR + n] =
+        const uint32_t gb = bf16_rne(v[0]), ub = bf16_rne(v[1]);
+        h[((int64_t)u * 2 + r) * I + (int64_t)it * kTR + n] =
             (uint16_t)bf16_rne(bf16_to_f32(glm_silu_bf16(gb)) * bf16_to_f32(ub));
     }
 };
@@ -1448,31 +1500,56 @@ template <int MR>
 static hipError_t union_gemvs(const MoeUnionArgs& a, hipStream_t st) {
     const int64_t rbH = row_bytes(T_Q4_K, a.H), rbI = row_bytes(T_Q4_K, a.I);
     const int itiles = (int)(a.I / kTR), htiles = (int)((a.H + kTR - 1) / kTR);
-    hipError_t e;
-    PlanS ps, psI;
-    if (MR == 2 && make_plans((int)(a.H / QK_K), ps) && make_plans((int)(a.I / QK_K), psI)) {
-        // two rows: gate and up of a tile in one workgroup, h written directly
-        const ProbUGateUpH ph{a.G, a.U, a.shG, a.shU, a.uidx, a.nslots, itiles, a.M, rbH, rbH * a.I, a.I, a.h};
-        e = runs_mr<2>(ph, ps, (unsigned)(a.max_slots * itiles), a.x, (int)a.H, st);
-    } else {
-        const ProbUGateUp<MR> pg{a.G, a.U, a.shG, a.shU, a.uidx, a.nslots, itiles, a.M, rbH, rbH * a.I, a.I, a.gu};
-        e = union_leg<MR>(pg, (int)(a.H / QK_K), (unsigned)(a.max_slots * 2 * itiles), a.x, (int)a.H, st);
-        if (e == hipSuccess) e = a.after_gateup(st);
-    }
+    const ProbUGateUp<MR> pg{a.G, a.U, a.shG, a.shU, a.uidx, a.nslots, itiles, a.M, rbH, rbH * a.I, a.I, a.gu};
+    hipError_t e = union_leg<MR>(pg, (int)(a.H / QK_K), (unsigned)(a.max_slots * 2 * itiles), a.x, (int)a.H, st);
+    if (e == hipSuccess) e = a.after_gateup(st);
     if (e != hipSuccess) return e;
+    PlanS psI;
     if (MR == 2 && make_plans((int)(a.I / QK_K), psI)) {
-        // two rows: kDownTiles tiles of the slot per workgroup
+        // one or two rows: kDownTiles tiles of the slot per workgroup
         const int htilesT = (htiles + kDownTiles - 1) / kDownTiles;
-        const ProbUDownT<kDownTiles> pd{a.D, a.shD, a.uidx, a.nslots, htilesT, a.M, rbI, rbI * a.H, a.I, a.H, a.h, a.y};
+        const ProbUDownT<kDownTiles> pd{a.D, a.shD, nullptr, a.uidx, a.nslots, htilesT, a.M, rbI, rbI * a.H, a.I, a.H,
+                                        a.h, a.y, {}};
         return runs_mr<2>(pd, psI, (unsigned)(a.max_slots * htilesT), a.h, (int)a.I, st);
     }
     const ProbUDown<MR> pd{a.D, a.shD, a.uidx, a.nslots, htiles, a.M, rbI, rbI * a.H, a.I, a.H, a.h, a.y};
     return union_leg<MR>(pd, (int)(a.I / QK_K), (unsigned)(a.max_slots * htiles), a.h, (int)a.I, st);
 }
 
-int moe_union_pass_rows(int64_t H, int64_t I) {
+// The pair legs' plan: where K does not split evenly, the last wave's part is short.  It copies and
+// multiplies whole blocks all the same (the bytes after its row: the next row's, or zero past the
+// tile), into block terms that no sum reads.  Covers every K up to 24 blocks (128 experts, 5632 x
+// 1792, top 8, M = 8, a single-row step per row before: 432 -> 210 us).
+static bool make_plans_pairs(int nsb, PlanS& p) {
+    if (make_plans(nsb, p)) return true;
+    for (int gs = 1; gs <= 3; ++gs) {
+        const int kp = (nsb + gs - 1) / gs;
+        const int64_t lds = (int64_t)kp * dma_bytes(gs);
+        if (kp > kMaxW || lds + (int64_t)kMaxW * gs * 1024 > kMaxLds1) continue;
+        p = PlanS{kp, gs, lds};
+        return true;
+    }
+    return false;
+}
+
+bool moe_pairs_supported(int64_t H, int64_t I) {
     PlanS p;
-    return make_plans((int)(H / QK_K), p) && make_plans((int)(I / QK_K), p) ? 2 : 8;
+    return I % kTR == 0 && make_plans_pairs((int)(H / QK_K), p) && make_plans_pairs((int)(I / QK_K), p);
+}
+
+hipError_t launch_moe_pairs_mfma(const MoePairArgs& a, hipStream_t st) {
+    PlanS psH, psI;
+    if (a.I % kTR != 0 || !make_plans_pairs((int)(a.H / QK_K), psH) || !make_plans_pairs((int)(a.I / QK_K), psI))
+        return hipErrorInvalidValue;
+    const int64_t rbH = row_bytes(T_Q4_K, a.H), rbI = row_bytes(T_Q4_K, a.I);
+    const int itiles = (int)(a.I / kTR), htiles = (int)((a.H + kTR - 1) / kTR);
+    const ProbUGateUpH pg{a.G, a.U, a.shG, a.shU, a.slots, a.nslots, itiles, a.M, rbH, rbH * a.I, a.I, a.h, {}};
+    const hipError_t e = runs_mr<2>(pg, psH, (unsigned)(a.max_slots * itiles), a.x, (int)a.H, st);
+    if (e != hipSuccess) return e;
+    const int htilesT = (htiles + kDownTiles - 1) / kDownTiles;
+    const ProbUDownT<kDownTiles> pd{a.D, a.shD, a.slots, nullptr, a.nslots, htilesT, 2, rbI, rbI * a.H, a.I, a.H,
+                                    a.h, a.y, {}};
+    return runs_mr<2>(pd, psI, (unsigned)(a.max_slots * htilesT), a.h, (int)a.I, st);
 }
 
 hipError_t launch_moe_union_mfma(const MoeUnionArgs& a, hipStream_t st) {

@@ -153,9 +153,21 @@ struct MoeUnionArgs {
     hipError_t after_gateup(hipStream_t st) const { return after_gateup_fn(*this, st); }
 };
 bool moe_union_supported(int64_t H, int64_t I, int M);
-// Rows per union pass: two when both legs fit the small-batch kernel (weights copied to LDS,
-// gate and up of a tile in one workgroup with the SwiGLU fused), else eight.
-int moe_union_pass_rows(int64_t H, int64_t I);
+// The same legs on slots of an expert and one or two of the rows that selected it, where both fit
+// the small-batch kernel (weights copied to LDS, gate and up of a tile in one workgroup with the
+// SwiGLU fused).  slots[u] = (expert or -1, row | row << 4 | two << 8).
+struct MoePairArgs {
+    const uint8_t *G, *U, *D, *shG, *shU, *shD;
+    const int2* slots;   // max_slots readable, *nslots valid
+    const int32_t* nslots;
+    int max_slots, M;
+    int64_t H, I;
+    const uint16_t* x;   // [M][H]
+    uint16_t* h;         // [slot][2][I]
+    uint16_t* y;         // [slot][2][H]
+};
+bool moe_pairs_supported(int64_t H, int64_t I);
+hipError_t launch_moe_pairs_mfma(const MoePairArgs& a, hipStream_t st);
 hipError_t launch_moe_union_mfma(const MoeUnionArgs& a, hipStream_t st);
 hipError_t launch_router_tail_rows(const uint16_t* logits, int M, int E, int topk, uint32_t scale_bits, int32_t* sel,
                                    uint16_t* selw, int32_t* sel2, uint16_t* selw2, hipStream_t st);

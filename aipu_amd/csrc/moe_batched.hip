@@ -7,12 +7,17 @@
 // facc += f32(gate * bf16(y_e)) only for the experts it selected, in ascending expert index,
 // then adds the shared expert with weight 1; fbuf = bf16(facc).
 //
-// Fast mode (Q4_K, up to 8 rows per pass, 2 where the union legs fit the small-batch
-// kernel): router logits for all rows, one routing decision per row, a one-wave union pass,
-// gate/up and down matrix-core GEMVs over the union slots (the grid is sized for the largest
-// possible union; workgroups past the live slot count return at once), h = bf16(silu(g) * u)
-// (fused into gate/up for two-row passes), and a per-row combine.  Reference mode runs each row
-// through the single-row reference path with its routing reordered by expert index.
+// Fast mode (Q4_K, up to 8 rows per pass): router logits for all rows, one routing decision per
+// row, the list of slots, gate/up and down matrix-core GEMVs over the slots (the grid is sized for
+// the largest possible list; workgroups past the live slot count return at once) and a per-row
+// combine.  Where the legs fit the small-batch kernel a slot is an expert with one or two of the
+// rows that selected it; otherwise an expert of the union with every row.  Reference mode runs each
+// row through the single-row reference path with its routing reordered by expert index.
+//
+// What bounds a pass: the weights of the union (57 of 256 experts for eight top-8 rows, 1.2 GB).
+// The pair slots replace passes of two rows over their own union each: those read 63 experts' worth
+// and paid router, routing, combine and both legs' ramps four times.  256 experts, 6144 x 2048, top
+// 8: M = 8 329 -> 240 us, M = 2 86.7 -> 83.5 us; 8 experts, 4096 x 1024, top 4, M = 8: 112 -> 45 us.
 #include "common.hpp"
 #include "glm_act.hpp"
 #include "launch.hpp"
@@ -24,6 +29,7 @@ namespace {
 constexpr int kRowsPerPass = 8;
 constexpr int64_t kAlign = 256;
 inline int64_t up(int64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
+constexpr int kUnionMaxE = 4096;            // experts of the fast step
 constexpr uint32_t kInactive = 0xFFFFFFFFu;   // no bf16-widened gate has this pattern
 
 int max_union_slots(int64_t E, int topk, bool shared) {
@@ -32,8 +38,18 @@ int max_union_slots(int64_t E, int topk, bool shared) {
 }
 
 struct BLayout {
-    int64_t logits, sel, selw, uidx, nslots, ugate, gu, h, y, single, total;
+    int64_t logits, sel, selw, uidx, nslots, ugate, slots, rslot, gu, h, y, single, total;
 };
+
+// Slots of one or two rows for M rows of topk distinct experts out of E: c rows of an expert take
+// (c + 1) / 2.  At most kRowsPerPass rows per union slot, so h and y hold them, too.
+int max_pair_slots(int M, int64_t E, int topk, bool shared) {
+    const int64_t n = (int64_t)M * topk, half = (M + 1) / 2;
+    int64_t u = (n + E) / 2;
+    if (u > n) u = n;
+    if (u > E * half) u = E * half;
+    return (int)(u + (shared ? half : 0));
+}
 
 BLayout b_layout(int64_t E, int64_t H, int64_t I, int topk) {
     const int ms = max_union_slots(E, topk, true);
@@ -45,6 +61,9 @@ BLayout b_layout(int64_t E, int64_t H, int64_t I, int topk) {
     L.uidx = o;   o += up((int64_t)ms * 4);
     L.nslots = o; o += up(4);
     L.ugate = o;  o += up((int64_t)kRowsPerPass * ms * 4);
+    const int mp = max_pair_slots(kRowsPerPass, E, topk, true);
+    L.slots = o;  o += up((int64_t)mp * 8);
+    L.rslot = o;  o += up((int64_t)kRowsPerPass * topk * 8);
     L.gu = o;     o += up((int64_t)ms * 2 * kRowsPerPass * I * 2);
     L.h = o;      o += up((int64_t)ms * kRowsPerPass * I * 2);
     L.y = o;      o += up((int64_t)ms * kRowsPerPass * H * 2);
@@ -59,7 +78,7 @@ BLayout b_layout(int64_t E, int64_t H, int64_t I, int topk) {
 __global__ __launch_bounds__(64) void k_union(const int32_t* __restrict__ sel, const uint16_t* __restrict__ selw,
                                               int M, int topk, int E, int shared, int ms, int32_t* __restrict__ uidx,
                                               int32_t* __restrict__ nslots, uint32_t* __restrict__ ugate) {
-    __shared__ uint8_t flag[4096];
+    __shared__ uint8_t flag[kUnionMaxE];
     __shared__ int32_t ulist[kRowsPerPass * 32];
     const int lane = threadIdx.x;
     for (int e = lane; e < E; e += 64) flag[e] = 0;
@@ -173,6 +192,156 @@ __global__ __launch_bounds__(kRUThreads) void k_route_union(const uint16_t* __re
     }
 }
 
+// The slots of M <= 8 rows, by one workgroup: experts in ascending index, each with its rows in
+// ascending order, two to a slot (slots[s] = (expert, row | row << 4 | two << 8)), then the shared
+// expert (-1) with all rows.  rslot[r * topk + k] = (2 * slot + half, gate) of row r's k-th
+// expert in ascending index; a slot of -1 is skipped.  The rows' decisions are in LDS.
+struct PairLists {
+    int2* slots;
+    int32_t* nslots;
+    int2* rslot;
+};
+__device__ __forceinline__ void list_pairs(const int32_t* s_sel, const uint16_t* s_selw, int M, int topk, int E,
+                                           int shared, uint32_t* s_mask, uint16_t* s_base, const PairLists& o) {
+    const int t = threadIdx.x, nthr = blockDim.x;
+    for (int j = t; j < E; j += nthr) s_mask[j] = 0u;
+    __syncthreads();
+    for (int j = t; j < M * topk; j += nthr) {
+        const int ej = s_sel[j];
+        if (ej >= 0 && ej < E) atomicOr(&s_mask[ej], 1u << (j / topk));
+    }
+    // the rank of selection i among its row's: the last threads first, while wave 0 numbers the slots
+    const int i = nthr - 1 - t, r = i / topk;   // M * topk <= 256 <= nthr
+    const bool mine = i < M * topk;
+    const int e = mine ? s_sel[i] : -1;
+    int rank = 0;
+    if (mine)
+        for (int k = r * topk; k < (r + 1) * topk; ++k) rank += s_sel[k] < e || (s_sel[k] == e && k < i);
+    __syncthreads();
+    if (t < 64) {   // 64 experts at a time; an expert's slots (0 .. 4) are counted bit by bit
+        const uint64_t below = (1ull << t) - 1ull;
+        int count = 0;
+        for (int c = 0; c < E; c += 64) {
+            const int ce = c + t;
+            uint32_t rows = ce < E ? s_mask[ce] : 0u;
+            const int need = (__popc(rows) + 1) >> 1;
+            const uint64_t n0 = __ballot(need & 1), n1 = __ballot(need & 2), n2 = __ballot(need & 4);
+            int s = count + __popcll(n0 & below) + 2 * __popcll(n1 & below) + 4 * __popcll(n2 & below);
+            if (ce < E) s_base[ce] = (uint16_t)s;
+            while (rows) {
+                const int r0 = __ffs(rows) - 1;
+                rows &= rows - 1u;
+                const int two = rows != 0u, r1 = two ? __ffs(rows) - 1 : r0;
+                rows &= rows - 1u;   // 0 stays 0
+                o.slots[s++] = make_int2(ce, r0 | r1 << 4 | two << 8);
+            }
+            count += __popcll(n0) + 2 * __popcll(n1) + 4 * __popcll(n2);
+        }
+        const int ns = shared ? (M + 1) / 2 : 0;
+        if (t < ns) {
+            const int two = 2 * t + 1 < M;
+            o.slots[count + t] = make_int2(-1, 2 * t | (2 * t + two) << 4 | two << 8);
+        }
+        if (t == 0) *o.nslots = count + ns;
+    }
+    __syncthreads();
+    if (mine) {
+        int2 v = make_int2(-1, (int)((uint32_t)s_selw[i] << 16));
+        if (e >= 0 && e < E) v.x = 2 * (int)s_base[e] + __popc(s_mask[e] & ((1u << r) - 1u));
+        o.rslot[r * topk + rank] = v;
+    }
+}
+
+// The routing of every row of a pass and its slots in one workgroup, for E <= kRouteMaxE: wave r
+// routes row r (route.hpp's decision on keys it forms itself, the winners and slot weights one per
+// lane), then list_pairs over the decisions held in LDS.
+__global__ __launch_bounds__(kRUThreads) void k_route_pairs(const uint16_t* __restrict__ logits, int M, int E, int topk,
+                                                            uint32_t scale_bits, int32_t* sel2, uint16_t* selw2,
+                                                            int shared, PairLists o) {
+    __shared__ int32_t s_sel[kRowsPerPass * kRouteMaxTopk];
+    __shared__ uint16_t s_selw[kRowsPerPass * kRouteMaxTopk];
+    __shared__ uint32_t s_mask[kRouteMaxE];
+    __shared__ uint16_t s_base[kRouteMaxE];
+    const int t = threadIdx.x, lane = t & 63;
+    const int r = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (r < M) {
+        uint32_t k[kRouteKeysPerLane];
+#pragma unroll
+        for (int j = 0; j < kRouteKeysPerLane; ++j) {
+            const int e = lane + 64 * j;
+            k[j] = e < E ? logits[(int64_t)r * E + e] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < kRouteKeysPerLane; ++j) {
+            const int e = lane + 64 * j;
+            k[j] = e < E ? route_key(k[j], e) : 0u;   // 0 is below every key
+        }
+        const uint32_t wl = route_tournament_lanes(k, topk, lane);
+        int32_t sl;
+        uint16_t swl;
+        route_weights_wave(wl, topk, scale_bits, lane, sl, swl);
+        if (lane < topk) {
+            const int i = r * topk + lane;
+            s_sel[i] = sl;
+            s_selw[i] = swl;
+            if (sel2) sel2[i] = sl;
+            if (selw2) selw2[i] = swl;
+        }
+    }
+    __syncthreads();
+    list_pairs(s_sel, s_selw, M, topk, E, shared, s_mask, s_base, o);
+}
+
+// The slots of decisions already in memory (E beyond kRouteMaxE).
+__global__ __launch_bounds__(256) void k_list_pairs(const int32_t* __restrict__ sel, const uint16_t* __restrict__ selw,
+                                                    int M, int E, int topk, int shared, PairLists o) {
+    __shared__ int32_t s_sel[kRowsPerPass * kRouteMaxTopk];
+    __shared__ uint16_t s_selw[kRowsPerPass * kRouteMaxTopk];
+    __shared__ uint32_t s_mask[kUnionMaxE];
+    __shared__ uint16_t s_base[kUnionMaxE];
+    for (int i = threadIdx.x; i < M * topk; i += blockDim.x) {
+        s_sel[i] = sel[i];
+        s_selw[i] = selw[i];
+    }
+    __syncthreads();
+    list_pairs(s_sel, s_selw, M, topk, E, shared, s_mask, s_base, o);
+}
+
+// out[m][d] = bf16(facc), facc over row m's own experts in ascending index, then the shared slot
+// with weight 1; resid (nullable) added after.  y [slot][2][H].  The outputs of up to eight experts
+// are loaded before their adds, so one memory round trip serves them.
+__global__ void k_pair_combine(const uint16_t* __restrict__ y, const int2* __restrict__ rslot, int topk,
+                               const int32_t* __restrict__ nslots, int shared, int M, int64_t H,
+                               const uint16_t* __restrict__ resid, uint16_t* __restrict__ out) {
+    constexpr int kChunk = 8;
+    const int m = blockIdx.y;
+    const int2* rs = rslot + m * topk;
+    const int sh = 2 * (*nslots - (M + 1) / 2) + m;   // half-slot of the shared expert
+    for (int64_t d = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; d < H; d += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t ysh = shared ? y[(int64_t)sh * H + d] : 0u;
+        float facc = 0.0f;
+        for (int k0 = 0; k0 < topk; k0 += kChunk) {
+            uint32_t yv[kChunk];
+            int2 s[kChunk];
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                s[k] = k0 + k < topk ? rs[k0 + k] : make_int2(-1, 0);
+                yv[k] = s[k].x >= 0 ? y[(int64_t)s[k].x * H + d] : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                if (s[k].x < 0) continue;
+                const float p = __uint_as_float((uint32_t)s[k].y) * bf16_to_f32(yv[k]);
+                facc = facc + p;
+            }
+        }
+        if (shared) facc = facc + bf16_to_f32(ysh);
+        uint32_t o = bf16_rne(facc);
+        if (resid) o = bf16_rne(bf16_to_f32(resid[m * H + d]) + bf16_to_f32(o));
+        out[m * H + d] = (uint16_t)o;
+    }
+}
+
 // h[u][m][i] = bf16(f32(glm_silu(g)) * f32(up)) for the live slots.
 __global__ void k_union_silu(const uint16_t* __restrict__ gu, const int32_t* __restrict__ nslots, int M, int64_t I,
                              int ms, uint16_t* __restrict__ h) {
@@ -191,7 +360,7 @@ __global__ void k_union_silu(const uint16_t* __restrict__ gu, const int32_t* __r
 
 // out[m][d] = bf16(facc), facc over the routed union slots in ascending expert index (only
 // the row's own experts), then the shared slot with weight 1; resid (nullable) added after.
-constexpr int kCombineChunk = 16;   // a two-row pass of top-8 routing has at most 16 union slots
+constexpr int kCombineChunk = 16;
 __global__ void k_union_combine(const uint16_t* __restrict__ y, const uint32_t* __restrict__ ugate,
                                 const int32_t* __restrict__ nslots, int shared, int M, int64_t H, int ms,
                                 const uint16_t* __restrict__ resid, int64_t rstride, uint16_t* __restrict__ out,
@@ -242,7 +411,63 @@ hipError_t after_gateup(const MoeUnionArgs& a, hipStream_t st) {
         if (e_ != hipSuccess) return e_;    \
     } while (0)
 
-// One fast pass over M <= 8 rows starting at row r0.
+// Router logits [M][E] of M <= 8 rows.
+hipError_t router_logits(const MoeArgs& a, const uint16_t* x, int M, uint16_t* logits, hipStream_t st) {
+    if (a.router_type == T_BF16)
+        return launch_router_bf16_logits_rows((const uint16_t*)a.router_w, x, a.H, (int)a.E, M, logits, st);
+    if (a.router_type == T_Q4_K && gemv_mfma_supported(a.E, a.H, M))
+        return launch_gemv_mfma(a.router_w, a.E, a.H, x, M, logits, nullptr, a.E, st);
+    if (a.router_type == T_Q4_K || gemv_mixed_supported(a.router_type, a.H))
+        return launch_gemv_fast(a.router_type, a.router_w, a.E, a.H, x, M, logits, nullptr, st);
+    // past the mixed-type kernel's staging limit: the exact kernel (within any tolerance)
+    return launch_gemv_ref(a.router_type, a.router_w, a.E, a.H, x, M, logits, nullptr, st);
+}
+
+// One fast pass over M <= 8 rows starting at row r0, on slots of one or two rows.
+hipError_t pair_pass(const MoeArgs& a, int64_t r0, int M, const BLayout& L, hipStream_t st) {
+    uint8_t* ws = (uint8_t*)a.ws;
+    uint16_t* logits = (uint16_t*)(ws + L.logits);
+    const uint16_t* x = a.x + r0 * a.H;
+    const int shared = a.sh_gate != nullptr ? 1 : 0;
+    AIPU_TRY(router_logits(a, x, M, logits, st));
+    int32_t* sel2 = a.sel_idx_out ? a.sel_idx_out + r0 * a.topk : nullptr;
+    uint16_t* selw2 = a.sel_w_out ? a.sel_w_out + r0 * a.topk : nullptr;
+    const PairLists o{(int2*)(ws + L.slots), (int32_t*)(ws + L.nslots), (int2*)(ws + L.rslot)};
+    if (a.E <= kRouteMaxE && a.topk <= kRouteMaxTopk) {
+        hipLaunchKernelGGL(k_route_pairs, dim3(1), dim3(kRUThreads), 0, st, logits, M, (int)a.E, a.topk, a.scale_bits,
+                           sel2, selw2, shared, o);
+    } else {
+        int32_t* sel = (int32_t*)(ws + L.sel);
+        uint16_t* selw = (uint16_t*)(ws + L.selw);
+        AIPU_TRY(launch_router_tail_rows(logits, M, (int)a.E, a.topk, a.scale_bits, sel, selw, sel2, selw2, st));
+        hipLaunchKernelGGL(k_list_pairs, dim3(1), dim3(256), 0, st, sel, selw, M, (int)a.E, a.topk, shared, o);
+    }
+    AIPU_TRY(hipGetLastError());
+    MoePairArgs u;
+    u.G = a.gate_exps;
+    u.U = a.up_exps;
+    u.D = a.down_exps;
+    u.shG = a.sh_gate;
+    u.shU = a.sh_up;
+    u.shD = a.sh_down;
+    u.slots = o.slots;
+    u.nslots = o.nslots;
+    u.max_slots = max_pair_slots(M, a.E, a.topk, shared);
+    u.M = M;
+    u.H = a.H;
+    u.I = a.I;
+    u.x = x;
+    u.h = (uint16_t*)(ws + L.h);
+    u.y = (uint16_t*)(ws + L.y);
+    AIPU_TRY(launch_moe_pairs_mfma(u, st));
+    int64_t b = (a.H + 255) / 256;
+    b = b > 1024 ? 1024 : b;
+    hipLaunchKernelGGL(k_pair_combine, dim3((unsigned)b, (unsigned)M), dim3(256), 0, st, u.y, o.rslot, a.topk, o.nslots,
+                       shared, M, a.H, a.resid ? a.resid + r0 * a.H : nullptr, a.y + r0 * a.H);
+    return hipGetLastError();
+}
+
+// One fast pass over M <= 8 rows starting at row r0, on the union of their experts.
 hipError_t fast_pass(const MoeArgs& a, int64_t r0, int M, const BLayout& L, hipStream_t st) {
     uint8_t* ws = (uint8_t*)a.ws;
     uint16_t* logits = (uint16_t*)(ws + L.logits);
@@ -254,17 +479,7 @@ hipError_t fast_pass(const MoeArgs& a, int64_t r0, int M, const BLayout& L, hipS
     const uint16_t* x = a.x + r0 * a.H;
     const bool shared = a.sh_gate != nullptr;
     const int ms = max_union_slots(a.E, a.topk, shared);
-
-    // router logits [M][E]
-    if (a.router_type == T_BF16) {
-        AIPU_TRY(launch_router_bf16_logits_rows((const uint16_t*)a.router_w, x, a.H, (int)a.E, M, logits, st));
-    } else if (a.router_type == T_Q4_K && gemv_mfma_supported(a.E, a.H, M)) {
-        AIPU_TRY(launch_gemv_mfma(a.router_w, a.E, a.H, x, M, logits, nullptr, a.E, st));
-    } else if (a.router_type == T_Q4_K || gemv_mixed_supported(a.router_type, a.H)) {
-        AIPU_TRY(launch_gemv_fast(a.router_type, a.router_w, a.E, a.H, x, M, logits, nullptr, st));
-    } else {   // past the mixed-type kernel's staging limit: the exact kernel (within any tolerance)
-        AIPU_TRY(launch_gemv_ref(a.router_type, a.router_w, a.E, a.H, x, M, logits, nullptr, st));
-    }
+    AIPU_TRY(router_logits(a, x, M, logits, st));
     int32_t* sel2 = a.sel_idx_out ? a.sel_idx_out + r0 * a.topk : nullptr;
     uint16_t* selw2 = a.sel_w_out ? a.sel_w_out + r0 * a.topk : nullptr;
     if (a.E <= kRouteMaxE && a.topk <= kRouteMaxTopk) {
@@ -311,21 +526,21 @@ int64_t moe_batched_workspace_bytes(int64_t E, int64_t H, int64_t I, int topk) {
 hipError_t launch_moe_decode_batched(const MoeArgs& a, int64_t M, hipStream_t st) {
     const BLayout L = b_layout(a.E, a.H, a.I, a.topk);
     uint8_t* ws = (uint8_t*)a.ws;
-    const bool fast = a.mode == AIPU_MODE_FAST && a.type == T_Q4_K && a.E <= 4096 && a.topk <= 32;
+    const bool fast = a.mode == AIPU_MODE_FAST && a.type == T_Q4_K && a.E <= kUnionMaxE && a.topk <= 32;
     if (M == 1) {   // the single-row step (slot-order combine, PE_M == 1)
         MoeArgs m = a;
         m.ws = ws + L.single;
         return launch_moe_decode(m, st);
     }
-    // passes of two rows where the union legs run on the small-batch kernel (fused SwiGLU):
-    // per row, two-row unions cost less than wider ones on the slower kernels
-    const int per = moe_union_pass_rows(a.H, a.I);
+    const bool pairs = moe_pairs_supported(a.H, a.I);
     int64_t r0 = 0;
     while (r0 < M) {
-        const int rows = (int)(M - r0 < per ? M - r0 : per);
-        // a leftover single row of the batch takes a one-row union pass too: the same kernels
-        // and summation order as the batch's other rows (the single-row step's legs differ)
-        if (fast && moe_union_supported(a.H, a.I, rows)) {
+        const int rows = (int)(M - r0 < kRowsPerPass ? M - r0 : kRowsPerPass);
+        // a leftover single row of the batch takes a one-row pass, too: the same kernels and
+        // summation order as the batch's other rows (the single-row step's legs differ)
+        if (fast && pairs) {
+            AIPU_TRY(pair_pass(a, r0, rows, L, st));
+        } else if (fast && moe_union_supported(a.H, a.I, rows)) {
             AIPU_TRY(fast_pass(a, r0, rows, L, st));
         } else {
             // one row at a time with its experts reordered by index (still the M > 1 order)

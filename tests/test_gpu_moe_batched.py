@@ -206,6 +206,24 @@ def test_batched_fast_two_row_pass_equals_one_row_pass(H, topk, shared):
     _check_fast(y2, sel2, sw2, X[:2], BF16, rw, ex, sh, E, H, I, topk)
 
 
+@pytest.mark.parametrize("M,E,topk,shared", [(7, 8, 8, True), (8, 4, 4, False), (9, 3, 2, True), (8, 600, 8, True)])
+def test_batched_fast_slot_lists(M, E, topk, shared):
+    """The slot lists of a pass at their limits: every row on every expert (four slots each, the
+    last one half empty at seven rows), fewer experts than rows, a leftover row, and routing outside
+    the one-workgroup kernel; within the fast-mode bound, and every row equal to a two-row batch."""
+    H, I = 512, 256
+    note(f"moe batched fast slot lists M={M} E={E} topk={topk} shared={shared}")
+    rng = np.random.default_rng(31 * M + E)
+    rw, ex, sh = _case(rng, E, H, I, BF16)
+    sh = sh if shared else None
+    X = qo.random_bf16(rng, (M, H), scale=0.05)
+    y, sel, sw = _run(BF16, rw, ex, sh, E, H, I, topk, X, "fast")
+    _check_fast(y, sel, sw, X, BF16, rw, ex, sh, E, H, I, topk)
+    for r in range(M):
+        y2, _, _ = _run(BF16, rw, ex, sh, E, H, I, topk, X[[r, (r + 1) % M]], "fast")
+        assert_bits_equal(y2[0], y[r], f"row {r}")
+
+
 def _random_batched_cases(n=10, seed=1505):
     """Seeded batched MoE shapes: M = 1..9 rows, E = topk..64 experts, H = 256..3072, I = 256..1536,
     top-1..8, bf16 or Q4_K router, with or without the shared expert."""
