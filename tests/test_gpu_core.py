@@ -102,12 +102,8 @@ def test_fp32_rsqrt_golden():
 
 
 # ------------------------------------------------------- reference-order GEMV
-# Q4_K runs on the register kernel (k_gemv_ref_q4k) while K * 4 bytes of staged activations fit
-# 128 KB, in passes of up to 8, 4, 2 or 1 rows as the staging allows: 9 rows at K = 256 (8 + 1),
-# 8 at K = 6144 (two passes of 4), 5 at K = 8192 (4 + 1), 2 at K = 32768 (one row per pass);
-# K = 40960 takes the staged-weights kernel.  Q8_0, F16 and BF16 take their register kernel
-# (k_gemv_ref_reg) at K a multiple of 64, Q6_K its own (k_gemv_ref_q6k, blocks alternately 4-B
-# aligned and 2 B past a dword) at K a multiple of 512 (K = 1280 stays on the staged kernel).
+# One kernel serves every type and K: passes of eight activation rows at most (9 rows at K = 256:
+# 8 + 1), Q6_K blocks alternately 4-B aligned and 2 B past a dword, long K (32768, 40960).
 # Ragged N leaves part of the last wave idle.
 REF_CASES = [
     (qo.GGML_Q4_K, 200, 768, 1), (qo.GGML_Q4_K, 131, 512, 3), (qo.GGML_Q4_K, 64, 256, 9),
