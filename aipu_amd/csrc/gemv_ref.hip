@@ -20,7 +20,7 @@
 // Stages of KS values of k go through a ring of three LDS buffers with one workgroup barrier per
 // stage: in interval t the producers write stage t and the chains add stage t - 2, reading ahead
 // into stage t - 1, which is complete already.
-// Measured (Q4_K, 6144 x 6144): M = 1 79 -> 23.5 us, M = 8 169 -> 45 us against one wave per 64 rows
+// Measured (Q4_K, 6144 x 6144): M = 1 80 -> 23.7 us, M = 8 171 -> 39.4 us against one wave per 64 rows
 // doing everything; the other types within a few us of these.
 // Any K (the last stage may be partial), any 2-byte aligned pointers (unaligned 16-B loads).
 #include "common.hpp"
