@@ -251,8 +251,8 @@ __device__ __forceinline__ void ref_rows(const uint8_t* __restrict__ W, int64_t 
             } else {
 #pragma unroll
                 for (int g = 0; g < C::G; ++g) {
-                    b.x[g][0] = load16_u2(xr[g] + 16 * r);
-                    b.x[g][1] = load16_u2(xr[g] + 16 * r + 8);
+                    b.x[g][0] = load16_u2(xr[g] + 16 * (int64_t)r);
+                    b.x[g][1] = load16_u2(xr[g] + 16 * (int64_t)r + 8);
                 }
             }
         };

@@ -231,6 +231,19 @@ def test_gemv_ref_row_split(t, N, K, M):
     assert_bits_equal(h_bits(y), ye, "y")
 
 
+def test_gemv_ref_k_beyond_2_31():
+    """A row of more than 2^31 weights: every offset into it and into the activations is 64-bit."""
+    K, M = (1 << 31) + 48, 2
+    note(f"gemv ref F16 K={K}")
+    w = torch.zeros(K, dtype=torch.float16, device="cuda")
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda")
+    for i, k in enumerate((0, 17, (1 << 30) + 5, (1 << 31) - 1, 1 << 31, K - 17, K - 1)):
+        w[k] = 1 << i
+        x[0, k], x[1, k] = 1.0, float(i)
+    _, yf = dev.gemv(qo.GGML_F16, w.view(torch.uint8), 1, K, x, mode="ref", out_f32=True)
+    assert yf.flatten().tolist() == [127.0, float(sum(i << i for i in range(7)))]
+
+
 def test_gemv_ref_full_north_star_shape():
     """K = N = 6144, M = 1: every output bit-exact against the C oracle."""
     note("gemv ref 6144x6144")
