@@ -720,7 +720,7 @@ hipError_t launch_gemv_fast(int type, const void* w, int64_t N, int64_t K, const
             // batch keep their one-row bits).  M = 1, streaming > matrix cores: K = 2048, N = 64 / 2048
             // 4.7 > 3.6 / 5.7 > 4.7 us; K = 6144, N = 256 / 2048 / 8192 7.3 > 7.7 / 10.7 > 9.8 / 34 > 21;
             // K = 8192, N = 512 / 8192 5.8 > 10.6 / 41 > 35.  M = 4 at 6144 x 6144: 86 > 17 us.
-            if (!(K <= 2560 || (K <= 6144 && N >= 2048)) || !gemv_mixed_supported(type, K))
+            if (!(K <= 2560 || (K <= 6144 && N >= 2048)) || N > kMixedMaxN || !gemv_mixed_supported(type, K))
                 return gemv_stream_mc<T_BF16, 2>((const uint8_t*)w, N, K, x, M, y, y_f32, st);
             [[fallthrough]];
         case T_Q6_K:

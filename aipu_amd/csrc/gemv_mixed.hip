@@ -46,6 +46,7 @@ using namespace mg;
 namespace {
 
 constexpr int kMixW = 4;                  // waves per workgroup (= K parts)
+static_assert(kMixedMaxN / kTR * kMixW * 64 <= 0xFFFFFFFFLL, "a grid's threads along x fit 32 bits");
 constexpr int kSliceBytes = 9 * 1024;     // per-wave weight slice: the largest group below
 
 // Bytes of one 256-weight block of one row in memory (kBlk) and in the LDS slice (kPitch),

@@ -546,7 +546,8 @@ int ref_rows_per_wg(int64_t rows, int cap) {
     return (int)(r < cap ? r : cap);
 }
 
-// One launch covers at most 2^26 rows and kMaxPasses passes of MC activation rows (grid limits).
+// One launch covers at most 2^26 rows and kMaxPasses passes of MC activation rows (a grid's threads
+// along x fit 32 bits).
 constexpr int64_t kMaxRows = 1LL << 26, kMaxPasses = 65535;
 
 template <int TYPE, int MC, int RM>
@@ -617,24 +618,37 @@ hipError_t launch_gemv_ref_tiles(const aipu_tile_desc* tiles, int n_tiles, int64
     for (int i = 0; i < n_tiles; ++i) rows += tiles[i].nrows;
     const auto run = [&](auto cfg, auto kernel, int mc, int rm) {
         typedef decltype(cfg) C;
+        // a launch's threads must fit 32 bits: pieces of at most kMaxRows rows, flushed before they exceed it
+        constexpr int64_t kMaxWgs = 0xFFFFFFFFLL / C::kThreads;
         const int R = ref_rows_per_wg(rows, rm);
         RefTiles a{};
         int64_t nwg = 0;
+        const auto flush = [&] {
+            for (int64_t m0 = 0; m0 < M && a.n; m0 += kMaxPasses * mc) {
+                const int64_t m = M - m0 < kMaxPasses * mc ? M - m0 : kMaxPasses * mc;
+                hipLaunchKernelGGL(kernel, dim3((unsigned)nwg, (unsigned)((m + mc - 1) / mc)), dim3(C::kThreads), C::kLds, st,
+                                   a, K, x + m0 * K, m, y + m0 * ys, y_f32 ? y_f32 + m0 * ys : nullptr, ys, R);
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess) return e;
+            }
+            a.n = 0;
+            nwg = 0;
+            return hipSuccess;
+        };
         for (int i = 0; i < n_tiles; ++i) {
             const aipu_tile_desc& d = tiles[i];
-            a.t[i] = RefTile{(const uint8_t*)d.w, d.row0, d.nrows, d.ggml_type, (int32_t)nwg};
-            nwg += (d.nrows + R - 1) / R;
-            if (nwg > (1LL << 30)) return hipErrorInvalidValue;
+            for (int64_t r0 = 0; r0 < d.nrows; r0 += kMaxRows) {
+                const int64_t n = d.nrows - r0 < kMaxRows ? d.nrows - r0 : kMaxRows, wgs = (n + R - 1) / R;
+                if (a.n == AIPU_MAX_TILES || nwg + wgs > kMaxWgs) {
+                    const hipError_t e = flush();
+                    if (e != hipSuccess) return e;
+                }
+                a.t[a.n++] = RefTile{(const uint8_t*)d.w + r0 * row_bytes(d.ggml_type, K), d.row0 + r0, n, d.ggml_type,
+                                     (int32_t)nwg};
+                nwg += wgs;
+            }
         }
-        a.n = n_tiles;
-        for (int64_t m0 = 0; m0 < M; m0 += kMaxPasses * mc) {
-            const int64_t m = M - m0 < kMaxPasses * mc ? M - m0 : kMaxPasses * mc;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)nwg, (unsigned)((m + mc - 1) / mc)), dim3(C::kThreads), C::kLds, st, a,
-                               K, x + m0 * K, m, y + m0 * ys, y_f32 ? y_f32 + m0 * ys : nullptr, ys, R);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
+        return flush();
     };
     if (M >= 5) return run(RefCfg<8, 32>{}, k_gemv_ref_tiles<8, 32>, 8, 32);
     if (M >= 3) return run(RefCfg<4, 32>{}, k_gemv_ref_tiles<4, 32>, 4, 32);

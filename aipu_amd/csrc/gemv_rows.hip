@@ -32,6 +32,8 @@ using namespace mg;
 namespace {
 
 constexpr int kRowMaxW = 8;                   // waves per workgroup
+constexpr int64_t kMaxN = 1LL << 26;          // rows of a launch: a grid's threads along x fit 32 bits
+static_assert(kMaxN / kTR * kRowMaxW * 64 <= 0xFFFFFFFFLL, "grid too large");
 constexpr int kNS = 2;                        // blocks in flight per wave
 constexpr int kSlot = 3 * 1024;               // 16 rows x 144 B in whole 1 KB copies
 // one activation row's operands of a block, [8 MFMAs][4 K-groups] 16 B, then its eight sub-block
@@ -282,7 +284,7 @@ hipError_t run_rows_any(const uint8_t* W, int64_t N, int nsb, const uint16_t* x,
 }  // namespace
 
 bool gemv_rows_supported(int64_t N, int64_t K, int M) {
-    if (M < 2 || M > 8 || N < 1 || K < QK_K || K % QK_K != 0 || K > (1 << 20)) return false;
+    if (M < 2 || M > 8 || N < 1 || N > kMaxN || K < QK_K || K % QK_K != 0 || K > (1 << 20)) return false;
     const int nsb = (int)(K / QK_K);
     return (M <= 2 ? rows_waves<2>(nsb) : M <= 4 ? rows_waves<4>(nsb) : rows_waves<8>(nsb)) > 0;
 }

@@ -54,7 +54,9 @@ hipError_t launch_gemv_tiles(const aipu_tile_desc* tiles, int n_tiles, int64_t N
                              int64_t M, uint16_t* y, float* y_f32, int mode, hipStream_t st);
 
 // gemv_mixed.hip -- one-launch GEMV over tiles of Q4_K / Q6_K / Q8_0 / F16 / BF16 rows
-// (tolerance mode, up to four activation rows per weight pass; row m of y at y + m * ys)
+// (tolerance mode, up to four activation rows per weight pass; row m of y at y + m * ys; a plain
+// GEMV of more than kMixedMaxN rows would not fit a grid)
+constexpr int64_t kMixedMaxN = 1LL << 27;
 bool gemv_mixed_supported(int type, int64_t K);
 hipError_t launch_gemv_mixed(const aipu_tile_desc* tiles, int n_tiles, int64_t K, const uint16_t* x, int64_t M,
                              uint16_t* y, float* y_f32, int64_t ys, hipStream_t st);

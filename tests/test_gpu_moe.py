@@ -646,6 +646,30 @@ def test_mixed_tiles_ref_one_launch(K, M, n_tiles, rows):
     assert np.all(gy[:, ~covered] == qo.bf16_round_bits(np.float32(7.0))), "rows outside the tiles written"
 
 
+def test_mixed_tiles_ref_beyond_one_grid():
+    """Tiles whose workgroups' threads do not fit one grid (2^28 rows at five activation rows) run in
+    several launches."""
+    K, M, n0 = 256, 5, 1 << 28
+    note(f"tiles ref {n0} rows")
+    rng = np.random.default_rng(28)
+    raw = qo.random_q4k_blocks(rng, 48)
+    w = torch.zeros(n0 * 144, dtype=torch.uint8, device="cuda")
+    at = [0, (1 << 26) - 8, 1 << 26, n0 - 8]   # eight rows each: both sides of a piece's end, the last rows
+    for i, r in enumerate(at):
+        w[r * 144:(r + 8) * 144] = d_u8(raw[i * 8 * 144:(i + 1) * 8 * 144])
+    tail = d_u8(raw[32 * 144:])
+    x = qo.random_bf16(rng, (M, K))
+    N = n0 + 16
+    y = torch.ones((M, N), dtype=torch.bfloat16, device="cuda")
+    dev.gemv_tiles([(Q4K, w, 0, n0), (Q4K, tail, n0, 16)], N, K, d_bf16(x), mode="ref", out=y)
+    _, ye = co.gemv_ref(Q4K, raw, 48, K, x)
+    ye = np.asarray(ye).reshape(M, 48)
+    for i, r in enumerate(at):
+        assert_bits_equal(h_bits(y[:, r:r + 8].contiguous()), ye[:, 8 * i:8 * i + 8], f"rows from {r}")
+    assert_bits_equal(h_bits(y[:, n0:].contiguous()), ye[:, 32:], "second tile")
+    assert int((y[:, :n0] != 0).sum()) <= M * 32
+
+
 def _tile_weights(rng, t, rows, K):
     """(raw bytes, dequantised float32[rows, K]) of a tile; BF16 tiles hold N(0, 0.05^2) bf16."""
     if t == BF16:
