@@ -61,10 +61,11 @@ BLayout b_layout(int64_t E, int64_t H, int64_t I, int topk) {
     L.uidx = o;   o += up((int64_t)ms * 4);
     L.nslots = o; o += up(4);
     L.ugate = o;  o += up((int64_t)kRowsPerPass * ms * 4);
-    const int mp = max_pair_slots(kRowsPerPass, E, topk, true);
-    L.slots = o;  o += up((int64_t)mp * 8);
-    L.rslot = o;  o += up((int64_t)kRowsPerPass * topk * 8);
     L.gu = o;     o += up((int64_t)ms * 2 * kRowsPerPass * I * 2);
+    // a pass on pair slots has no gu: its lists (at most 4 ms slots of 8 bytes, 8 topk entries) fit there
+    // from I = 256 on, and the workspace stays the size that callers may have kept
+    L.slots = L.gu;
+    L.rslot = L.slots + up((int64_t)max_pair_slots(kRowsPerPass, E, topk, true) * 8);
     L.h = o;      o += up((int64_t)ms * kRowsPerPass * I * 2);
     L.y = o;      o += up((int64_t)ms * kRowsPerPass * H * 2);
     L.single = o; o += moe_workspace_bytes(E, H, I, topk);   // reference path, one row at a time

@@ -146,6 +146,13 @@ def test_moe_validation():
     assert f2(12, FAKE, FAKE, FAKE, 500, 256, FAKE, FAKE, NULL, 1, FAKE, 10, S) == SHAPE
 
 
+@pytest.mark.parametrize("E,H,I,topk,n", [(1, 256, 256, 1, 40192), (8, 4096, 1024, 4, 1122816), (256, 6144, 2048, 8, 13033984),
+                                          (4096, 512, 256, 32, 5435648), (64, 1024, 512, 32, 2841856)])
+def test_batched_workspace_keeps_its_size(E, H, I, topk, n):
+    """A caller's buffer of the documented size is never too small for a later build."""
+    assert L().aipu_moe_batched_workspace_bytes(E, H, I, topk) <= n
+
+
 def test_prefill_validation():
     f = L().aipu_gemm_prefill
     wsb = L().aipu_gemm_prefill_workspace_bytes
