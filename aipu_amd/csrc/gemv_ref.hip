@@ -13,15 +13,15 @@
 // consecutive weights of one row) and writes to LDS, four consecutive k per 16-B slot, neighbouring
 // rows in neighbouring slots.  What it writes depends on what is scarce:
 //   * One or two activation rows: the products x * w, so that the chain is a read and four adds per
-//     four k (the read hides behind the adds' latency; 10 cycles per k measured).
-//   * More: the weights, with the stage's activations as fp32 beside them, and the chain multiplies.
-//     A chain wave then takes 15 cycles per k, but the producers, whose products of eight rows took
-//     28 cycles per k, write each weight once (M = 8 at 6144 x 6144: 82 -> 47 us).
+//     four k (the reads hide behind the adds' latency).
+//   * More: the weights, with the stage's activations as fp32 beside them, and the chain multiplies,
+//     so that the producers convert and write each weight once.
 // Stages of KS values of k go through a ring of three LDS buffers with one workgroup barrier per
 // stage: in interval t the producers write stage t and the chains add stage t - 2, reading ahead
 // into stage t - 1, which is complete already.
-// Measured (Q4_K, 6144 x 6144): M = 1 80 -> 23.7 us, M = 8 171 -> 39.4 us against one wave per 64 rows
-// doing everything; the other types within a few us of these.
+// Measured (Q4_K, 6144 x 6144), one wave per 64 rows doing everything -> here: M = 1 / 2 / 4 / 8
+// 79 / 111 / 166 / 167 -> 23 / 26 / 39 / 39 us; the other types within a few us of these.  At many rows the chain
+// is not what binds, and that one wave is the faster one (k_gemv_ref_wave, ref_wave_wins).
 // Any K (the last stage may be partial), any 2-byte aligned pointers (unaligned 16-B loads).
 #include "common.hpp"
 #include "launch.hpp"
@@ -411,6 +411,211 @@ __device__ __forceinline__ void ref_rows(const uint8_t* __restrict__ W, int64_t 
     }
 }
 
+// ---------------------------------------------------------------- one wave per 64 rows
+// At many rows the chain is not what binds: workgroups of ref_rows share a CU's VALU and LDS, and a
+// product costs there a second conversion of the activations and 4 bytes written and read.  Here one
+// wave owns 64 rows and does everything: lane = row, a unit of the row's weights in registers, loaded
+// one unit ahead, the activations as fp32 in LDS, converted once for the 64 rows.  About five VALU
+// operations per weight and one more pair per further activation row; slower alone (6144 x 6144:
+// 79 us against 23) and faster once it fills the chip.  A unit is 256 weights (Q4_K: 9 16-B pieces;
+// Q6_K: the 53 dwords that span a 210-B block, which starts 4-B aligned or 2 bytes past) or 64 (Q8_0:
+// 17 dwords; F16 / BF16: 8 16-B pieces).
+constexpr int kWaveChunk = 256;   // activations staged at a time
+
+// A unit: load() fetches it, each() calls f(c, weight) for its weights 4 c .. 4 c + 3 in order, weight(e)
+// dequantising weight 4 c + e exactly as the reference does.
+template <int TYPE>
+struct Unit;
+
+template <>
+struct Unit<T_Q4_K> {
+    static constexpr int kW = 256, kBytes = 144;
+    uint4 r[9];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t wr, uint32_t o) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) r[i] = buf_load16(wr, o + 16u * (uint32_t)i);
+    }
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t, F f) const {
+        const float d = f16_to_f32(r[0].x & 0xFFFFu), dm = f16_to_f32(r[0].x >> 16);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            uint32_t sc, mn;
+            q4k_scale_min(j, r[0].y, r[0].z, r[0].w, sc, mn);
+            const float D = d * (float)sc, Mn = dm * (float)mn;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const uint32_t x = word_of(r[1 + 2 * (j >> 1) + (c >> 2)], c & 3);
+                const uint32_t v = ((j & 1) ? x >> 4 : x) & 0x0F0F0F0Fu;
+                const float q[4] = {cvt_ubyte<0>(v), cvt_ubyte<1>(v), cvt_ubyte<2>(v), cvt_ubyte<3>(v)};
+                f(8 * j + c, [&](int e) { return __builtin_fmaf(D, q[e], -Mn); });   // D * q is exact
+            }
+        }
+    }
+};
+
+template <>
+struct Unit<T_Q6_K> {
+    static constexpr int kW = 256, kBytes = 210;
+    uint32_t r[53];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t wr, uint32_t o) {   // o: the dword the block starts in
+#pragma unroll
+        for (int i = 0; i < 53; ++i) r[i] = buf_load4(wr, o + 4u * (uint32_t)i);
+    }
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t par, F f) const {   // the block starts par (0 or 2) bytes into r[0]
+        const auto dw = [&](int o) { return __builtin_amdgcn_alignbyte(r[(o >> 2) + 1], r[o >> 2], par); };
+        const float d = f16_to_f32(par ? r[52] >> 16 : r[52] & 0xFFFFu);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                __builtin_amdgcn_sched_barrier(0);   // one run of 32 weights at a time (registers)
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    const uint32_t ql = dw(64 * h + 32 * (t & 1) + 4 * c), qh = dw(128 + 32 * h + 4 * c);
+                    const uint32_t code = ((t < 2 ? ql : ql >> 4) & 0x0F0F0F0Fu) | (((qh >> (2 * t)) & 0x03030303u) << 4);
+                    const int si = 8 * h + 2 * t + (c >> 2);
+                    const float ds = d * (float)(int8_t)(uint8_t)(dw(192 + (si & ~3)) >> (8 * (si & 3)));
+                    const float q[4] = {cvt_ubyte<0>(code), cvt_ubyte<1>(code), cvt_ubyte<2>(code), cvt_ubyte<3>(code)};
+                    f(32 * h + 8 * t + c, [&](int e) { return ds * (q[e] - 32.0f); });
+                }
+            }
+    }
+};
+
+template <>
+struct Unit<T_Q8_0> {
+    static constexpr int kW = 64, kBytes = 68;
+    uint32_t r[17];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t wr, uint32_t o) {
+#pragma unroll
+        for (int i = 0; i < 17; ++i) r[i] = buf_load4(wr, o + 4u * (uint32_t)i);
+    }
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t, F f) const {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const float d = f16_to_f32(c < 8 ? r[0] & 0xFFFFu : r[8] >> 16);
+            f(c, [&](int e) {
+                const int b = (c < 8 ? 2 : 4) + 4 * c + e;   // byte of the unit: 2 of each block's d lie before it
+                return d * (float)(int8_t)(uint8_t)(r[b >> 2] >> (8 * (b & 3)));
+            });
+        }
+    }
+};
+
+template <int TYPE>
+struct UnitHalf {   // F16 / BF16
+    static constexpr int kW = 64, kBytes = 128;
+    uint4 r[8];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t wr, uint32_t o) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = buf_load16(wr, o + 16u * (uint32_t)i);
+    }
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t, F f) const {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            f(c, [&](int e) {
+                const uint32_t h = word_of(r[c >> 1], 2 * (c & 1) + (e >> 1)) >> (16 * (e & 1)) & 0xFFFFu;
+                return TYPE == T_F16 ? f16_to_f32(h) : bf16_to_f32(h);
+            });
+        }
+    }
+};
+template <>
+struct Unit<T_F16> : UnitHalf<T_F16> {};
+template <>
+struct Unit<T_BF16> : UnitHalf<T_BF16> {};
+
+// Rows [row0, row0 + 64) of W [N][K] against activation rows X [mcnt][K], K a multiple of 64;
+// y[m * ys + row].  s_x: [2][MC][kWaveChunk].
+template <int TYPE, int MC>
+__device__ __forceinline__ void ref_wave(const uint8_t* __restrict__ W, int64_t N, int64_t K,
+                                         const uint16_t* __restrict__ X, int mcnt, uint16_t* __restrict__ Y,
+                                         float* __restrict__ Yf, int64_t ys, int64_t row0, float* s_x) {
+    typedef Unit<TYPE> U;
+    constexpr int kPer = kWaveChunk / U::kW;   // units per chunk
+    const int lane = threadIdx.x;
+    const int nu = (int)(K / U::kW), nch = (nu + kPer - 1) / kPer;
+    const uint32_t rb = (uint32_t)row_bytes(TYPE, K);
+    const int nrows = (int)(N - row0 < 64 ? N - row0 : 64);
+    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W + row0 * (int64_t)rb, (uint32_t)nrows * rb);   // rows past N read zeros
+    const uint32_t wrow = (uint32_t)lane * rb;
+    const auto load = [&](U& u, int i) {   // Q6_K: the dwords that span the block (the last may reach past the row)
+        const uint32_t o = (uint32_t)U::kBytes * (uint32_t)i;
+        u.load(wr, wrow + (TYPE == T_Q6_K ? o & ~3u : o));
+    };
+    // a chunk's activations: four per lane and row, past K the last ones (not used)
+    uint2 xv[MC];
+    const uint16_t* xr[MC];
+#pragma unroll
+    for (int m = 0; m < MC; ++m) xr[m] = X + (int64_t)(m < mcnt ? m : mcnt - 1) * K;
+    const auto fetch = [&](int c) {
+        int64_t k = (int64_t)c * kWaveChunk + 4 * lane;
+        k = k + 4 <= K ? k : K - 4;
+#pragma unroll
+        for (int m = 0; m < MC; ++m) xv[m] = *(const uint2*)(xr[m] + k);
+    };
+    const auto stage = [&](int buf) {
+#pragma unroll
+        for (int m = 0; m < MC; ++m)
+            *(float4*)(s_x + (buf * MC + m) * kWaveChunk + 4 * lane) =
+                make_float4(bf16_to_f32(xv[m].x & 0xFFFFu), __uint_as_float(xv[m].x & 0xFFFF0000u),
+                            bf16_to_f32(xv[m].y & 0xFFFFu), __uint_as_float(xv[m].y & 0xFFFF0000u));
+    };
+    float acc[MC];
+#pragma unroll
+    for (int m = 0; m < MC; ++m) acc[m] = 0.0f;
+    U cur, nxt;
+    fetch(0);
+    load(nxt, 0);
+    stage(0);
+    fetch(1);
+    int i = 0;
+    for (int c = 0; c < nch; ++c) {
+        // the next chunk (past K: repeated values) goes to the other buffer before this one is used: no wait
+        // between chunks, and no barrier for one wave, whose LDS accesses are in order; a branch around
+        // the last chunk's staging cost up to 6 %
+        stage((c + 1) & 1);
+        fetch(c + 2);
+        __builtin_amdgcn_wave_barrier();
+        const float* xb = s_x + (c & 1) * (MC * kWaveChunk);
+        const int n = kPer == 1 ? 1 : nu - i < kPer ? nu - i : kPer;
+        for (int u = 0; u < n; ++u, ++i) {
+            cur = nxt;
+            if (i + 1 < nu) load(nxt, i + 1);
+            const float* xu = xb + u * U::kW;
+            cur.each(((uint32_t)U::kBytes * (uint32_t)i) & 3u, [&](int q, auto weight) {
+                constexpr bool kFirst = TYPE == T_Q8_0 && MC == 2;   // weights before the reads: 42 -> 38 us (16384 x 2048)
+                float wf[4];
+                if (kFirst)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) wf[e] = weight(e);
+                float4 x[MC];
+#pragma unroll
+                for (int m = 0; m < MC; ++m) x[m] = *(const float4*)(xu + m * kWaveChunk + 4 * q);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float w = kFirst ? wf[e] : weight(e);
+#pragma unroll
+                    for (int m = 0; m < MC; ++m) {
+                        const float p = (e == 0 ? x[m].x : e == 1 ? x[m].y : e == 2 ? x[m].z : x[m].w) * w;
+                        acc[m] = acc[m] + p;
+                    }
+                }
+            });
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (lane < nrows)
+        for (int m = 0; m < mcnt; ++m) {
+            Y[(int64_t)m * ys + row0 + lane] = (uint16_t)bf16_rne(acc[m]);
+            if (Yf) Yf[(int64_t)m * ys + row0 + lane] = acc[m];
+        }
+}
+
 // Slot gathering (MoE): blockIdx.z = slot z reads weight matrix sel[z] of the `_exps`
 // stack at W + sel[z]*wstride when z < topk, else W_alt (the shared expert); activations
 // and outputs are offset by z*x_zstride / z*y_zstride.  Slots nslots .. 2 nslots - 1 are the same
@@ -430,36 +635,49 @@ struct RefGather {
     int64_t y_zstride;
 };
 
-template <int TYPE, int MC, int RM>
-__global__ __launch_bounds__((RefCfg<MC, RM>::kThreads)) void k_gemv_ref(const uint8_t* __restrict__ W, int64_t N, int64_t K,
-                                                                         const uint16_t* __restrict__ X, int64_t M,
-                                                                         uint16_t* __restrict__ Y, float* __restrict__ Yf,
-                                                                         int64_t ys, int R, RefGather ga) {
-    extern __shared__ __align__(16) uint8_t s_ref[];
-    if (ga.sel) {
-        int z = blockIdx.z;
-        const uint8_t* alt = ga.W_alt;
-        if (z >= ga.nslots) {
-            z -= ga.nslots;
-            W = ga.W2;
-            alt = ga.W2_alt;
-            Y = ga.Y2;
-        }
-        if (z < ga.topk) {
-            int e = ga.sel[z];
-            e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
-            W += (int64_t)e * ga.wstride;
-        } else {
-            W = alt;
-        }
-        X += (int64_t)z * ga.x_zstride;
-        Y += (int64_t)z * ga.y_zstride;
-        if (Yf) Yf += (int64_t)z * ga.y_zstride;
+__device__ __forceinline__ void ref_gather(const RefGather& ga, const uint8_t*& W, const uint16_t*& X, uint16_t*& Y,
+                                           float*& Yf) {
+    if (!ga.sel) return;
+    int z = blockIdx.z;
+    const uint8_t* alt = ga.W_alt;
+    if (z >= ga.nslots) {
+        z -= ga.nslots;
+        W = ga.W2;
+        alt = ga.W2_alt;
+        Y = ga.Y2;
     }
+    if (z < ga.topk) {
+        int e = ga.sel[z];
+        e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
+        W += (int64_t)e * ga.wstride;
+    } else {
+        W = alt;
+    }
+    X += (int64_t)z * ga.x_zstride;
+    Y += (int64_t)z * ga.y_zstride;
+    if (Yf) Yf += (int64_t)z * ga.y_zstride;
+}
+
+template <int TYPE, int MC, int RM>
+__global__ __launch_bounds__((RefCfg<MC, RM>::kThreads)) void k_gemv_ref(const uint8_t* W, int64_t N, int64_t K,
+                                                                         const uint16_t* X, int64_t M, uint16_t* Y,
+                                                                         float* Yf, int64_t ys, int R, RefGather ga) {
+    extern __shared__ __align__(16) uint8_t s_ref[];
+    ref_gather(ga, W, X, Y, Yf);
     const int64_t m0 = (int64_t)blockIdx.y * MC;
     const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
     ref_rows<TYPE, MC, RM>(W, N, K, X + m0 * K, mcnt, Y + m0 * ys, Yf ? Yf + m0 * ys : nullptr, ys,
                            (int64_t)blockIdx.x * R, R, s_ref);
+}
+
+template <int TYPE, int MC>
+__global__ __launch_bounds__(64) void k_gemv_ref_wave(const uint8_t* W, int64_t N, int64_t K, const uint16_t* X, int64_t M,
+                                                      uint16_t* Y, float* Yf, int64_t ys, RefGather ga) {
+    __shared__ __align__(16) float s_x[2 * MC * kWaveChunk];
+    ref_gather(ga, W, X, Y, Yf);
+    const int64_t m0 = (int64_t)blockIdx.y * MC;
+    const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
+    ref_wave<TYPE, MC>(W, N, K, X + m0 * K, mcnt, Y + m0 * ys, Yf ? Yf + m0 * ys : nullptr, ys, (int64_t)blockIdx.x * 64, s_x);
 }
 
 // A tile sequence of mixed types in one launch: workgroup g belongs to the last tile whose wg0 is
@@ -550,24 +768,13 @@ int ref_rows_per_wg(int64_t rows, int cap) {
 // along x fit 32 bits).
 constexpr int64_t kMaxRows = 1LL << 26, kMaxPasses = 65535;
 
-template <int TYPE, int MC, int RM>
-hipError_t run_ref(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int64_t M, uint16_t* y, float* y_f32,
-                   int nslots, const RefGather& ga, hipStream_t st) {
-    typedef RefCfg<MC, RM> C;
-    const int R = ref_rows_per_wg(N * nslots, RM);
-    for (int64_t m0 = 0; m0 < M; m0 += kMaxPasses * MC) {
-        const int64_t m = M - m0 < kMaxPasses * MC ? M - m0 : kMaxPasses * MC;
+// Calls fn(n0, n, m0, m) for pieces of at most kMaxRows rows and kMaxPasses passes.
+template <class F>
+hipError_t for_pieces(int64_t N, int64_t M, int mc, F fn) {
+    for (int64_t m0 = 0; m0 < M; m0 += kMaxPasses * mc) {
+        const int64_t m = M - m0 < kMaxPasses * mc ? M - m0 : kMaxPasses * mc;
         for (int64_t n0 = 0; n0 < N; n0 += kMaxRows) {   // slots (nslots > 1): N is an expert's row count
-            const int64_t n = N - n0 < kMaxRows ? N - n0 : kMaxRows;
-            const dim3 grid((unsigned)((n + R - 1) / R), (unsigned)((m + MC - 1) / MC), (unsigned)nslots);
-            RefGather g = ga;
-            if (g.W_alt) g.W_alt += n0 * row_bytes(TYPE, K);
-            if (g.W2) g.W2 += n0 * row_bytes(TYPE, K);
-            if (g.W2_alt) g.W2_alt += n0 * row_bytes(TYPE, K);
-            if (g.Y2) g.Y2 += n0;
-            hipLaunchKernelGGL((k_gemv_ref<TYPE, MC, RM>), grid, dim3(C::kThreads), C::kLds, st,
-                               W + n0 * row_bytes(TYPE, K), n, K, x + m0 * K, m, y + m0 * N + n0,
-                               y_f32 ? y_f32 + m0 * N + n0 : nullptr, N, R, g);
+            fn(n0, N - n0 < kMaxRows ? N - n0 : kMaxRows, m0, m);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
@@ -575,15 +782,116 @@ hipError_t run_ref(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, in
     return hipSuccess;
 }
 
+RefGather gather_from(RefGather g, int64_t n0, int64_t rb) {
+    if (g.W_alt) g.W_alt += n0 * rb;
+    if (g.W2) g.W2 += n0 * rb;
+    if (g.W2_alt) g.W2_alt += n0 * rb;
+    if (g.Y2) g.Y2 += n0;
+    return g;
+}
+
+struct RefCall {
+    const uint8_t* W;
+    int64_t N, K;
+    const uint16_t* x;
+    int64_t M;
+    uint16_t* y;
+    float* y_f32;
+    int64_t ys;
+    int nslots;
+    RefGather ga;
+    hipStream_t st;
+};
+
+template <int TYPE, int MC, int RM>
+hipError_t run_ref(const RefCall& c) {
+    typedef RefCfg<MC, RM> C;
+    const int R = ref_rows_per_wg(c.N * c.nslots * ((c.M + MC - 1) / MC), RM);
+    const int64_t rb = row_bytes(TYPE, c.K);
+    return for_pieces(c.N, c.M, MC, [&](int64_t n0, int64_t n, int64_t m0, int64_t m) {
+        const dim3 grid((unsigned)((n + R - 1) / R), (unsigned)((m + MC - 1) / MC), (unsigned)c.nslots);
+        hipLaunchKernelGGL((k_gemv_ref<TYPE, MC, RM>), grid, dim3(C::kThreads), C::kLds, c.st, c.W + n0 * rb, n, c.K,
+                           c.x + m0 * c.K, m, c.y + m0 * c.ys + n0, c.y_f32 ? c.y_f32 + m0 * c.ys + n0 : nullptr, c.ys, R,
+                           gather_from(c.ga, n0, rb));
+    });
+}
+
+template <int TYPE, int MC>
+hipError_t run_ref_wave(const RefCall& c) {
+    // 16-bit rows at two activation rows: four waves per CU where more would thrash the rows' lines (200000 x
+    // 6144: 661 -> 578 us; 72000 x 6144, whose waves all fit, 198 -> 273)
+    const bool few = (TYPE == T_F16 || TYPE == T_BF16) && MC == 2 && c.K >= 2048 &&
+                     c.N * c.nslots * ((c.M + MC - 1) / MC) >= 440 * (int64_t)device_cu_count();
+    const int pad = few ? 40 * 1024 - 2 * MC * kWaveChunk * 4 : 0;
+    const int64_t rb = row_bytes(TYPE, c.K);
+    return for_pieces(c.N, c.M, MC, [&](int64_t n0, int64_t n, int64_t m0, int64_t m) {
+        const dim3 grid((unsigned)((n + 63) / 64), (unsigned)((m + MC - 1) / MC), (unsigned)c.nslots);
+        hipLaunchKernelGGL((k_gemv_ref_wave<TYPE, MC>), grid, dim3(64), pad, c.st, c.W + n0 * rb, n, c.K, c.x + m0 * c.K, m,
+                           c.y + m0 * c.ys + n0, c.y_f32 ? c.y_f32 + m0 * c.ys + n0 : nullptr, c.ys,
+                           gather_from(c.ga, n0, rb));
+    });
+}
+
+// Whether the one-wave kernel takes these pointers and this K (whole units, its loads' alignment).
+bool ref_wave_takes(int type, const RefCall& c) {
+    const uintptr_t wa = type == T_Q8_0 || type == T_Q6_K ? 4 : 16;
+    const auto al = [](const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; };
+    return c.K % (type == T_Q6_K ? 512 : type == T_Q4_K ? 256 : 64) == 0 && c.K <= (1 << 20) && al(c.x, 8) && al(c.W, wa) &&
+           al(c.ga.W_alt, wa) && al(c.ga.W2, wa) && al(c.ga.W2_alt, wa) && c.ga.x_zstride % 4 == 0 &&
+           c.ga.wstride % (int64_t)wa == 0;
+}
+
+// Whether the one-wave kernel is the faster one for `rows` rows (of all slots, times the passes of
+// activation rows).  ref_rows takes a time that grows with the rows once every CU has a workgroup, in
+// steps of 32 rows per CU; the one-wave kernel takes the same time up to 64 rows per SIMD.  The lines
+// cross at these rows per CU, earlier where K is short and ref_rows' stages are few.  Q4_K, K = 6144,
+// ref_rows > one wave: M = 1, 32768 / 65536 / 154880 rows 62 > 74 / 115 > 75 / 282 > 141 us; M = 2, 24576 /
+// 32768 / 65536 rows 90 > 100 / 118 > 101 / 230 > 105 us; M = 4, 49152 / 65536 rows 156 > 172 / 208 > 177 us;
+// M = 8, 65536 / 98304 rows 262 > 300 / 389 > 340 us.  Q8_0 and the 16-bit types, whose rows the one-wave
+// kernel reads 68 or 128 bytes at a time, stay on ref_rows at M = 1 and M = 8 (Q8_0: 131072 rows 345 and
+// 415 us at M = 1, 154880 rows 616 and 735 us at M = 8), but for a short K, and 16 bits
+// from 130 rows per CU to 256 or 400 at M = 1 and K <= 2048 (200000 x 1024: 72 and 97 us).
+bool ref_wave_wins(int type, int64_t rows, int64_t M, int64_t K) {
+    const int per = (int)(rows / device_cu_count() < 1 << 20 ? rows / device_cu_count() : 1 << 20);
+    const int i = M >= 5 ? 3 : M >= 3 ? 2 : (int)M - 1;
+    if (type == T_Q4_K) {
+        const int at[4] = {K <= 256 ? 104 : 130, K <= 512 ? 64 : 97, K <= 512 ? 130 : 194, K <= 256 ? 208 : K <= 512 ? 256 : 288};
+        return per >= at[i];
+    }
+    if (type == T_Q6_K) {
+        const int at[4] = {66, K <= 512 ? 56 : 66, K <= 512 ? 130 : 192, K <= 512 ? 224 : 300};
+        return per >= at[i];
+    }
+    if (i == 0) return K <= 256 ? per >= 120 : type != T_Q8_0 && K <= 2048 && per >= 130 && per < (K <= 1024 ? 400 : 256);
+    if (i == 1) return per >= (K <= 512 ? 64 : type != T_Q8_0 && K >= 4096 ? 130 : 97);
+    if (i == 2) return per >= (K <= 512 ? 130 : K > 8192 ? 256 : 194);
+    return K <= 256 ? per >= 232 : K <= 512 && per >= 380;
+}
+
 template <int TYPE>
-hipError_t run_ref_type(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int64_t M, uint16_t* y,
-                        float* y_f32, int nslots, const RefGather& ga, hipStream_t st) {
-    if (M >= 5) return run_ref<TYPE, 8, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-    if (M >= 3) return run_ref<TYPE, 4, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-    if (M == 2) return run_ref<TYPE, 2, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-    if (N * nslots <= 32 * (int64_t)device_cu_count())
-        return run_ref<TYPE, 1, 32>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-    return run_ref<TYPE, 1, 64>(W, N, K, x, M, y, y_f32, nslots, ga, st);
+hipError_t run_ref_type(const RefCall& c) {
+    const int64_t M = c.M, mc = M >= 5 ? 8 : M >= 3 ? 4 : M;
+    if (ref_wave_takes(TYPE, c) && ref_wave_wins(TYPE, c.N * c.nslots * ((M + mc - 1) / mc), M, c.K)) {
+        if (M >= 5) return run_ref_wave<TYPE, 8>(c);
+        if (M >= 3) return run_ref_wave<TYPE, 4>(c);
+        return M == 2 ? run_ref_wave<TYPE, 2>(c) : run_ref_wave<TYPE, 1>(c);
+    }
+    if (M >= 5) return run_ref<TYPE, 8, 32>(c);
+    if (M >= 3) return run_ref<TYPE, 4, 32>(c);
+    if (M == 2) return run_ref<TYPE, 2, 32>(c);
+    if (c.N * c.nslots <= 32 * (int64_t)device_cu_count()) return run_ref<TYPE, 1, 32>(c);
+    return run_ref<TYPE, 1, 64>(c);
+}
+
+hipError_t run_ref_any(int type, const RefCall& c) {
+    switch (type) {
+        case T_Q4_K: return run_ref_type<T_Q4_K>(c);
+        case T_Q6_K: return run_ref_type<T_Q6_K>(c);
+        case T_Q8_0: return run_ref_type<T_Q8_0>(c);
+        case T_F16: return run_ref_type<T_F16>(c);
+        case T_BF16: return run_ref_type<T_BF16>(c);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace
@@ -592,18 +900,9 @@ hipError_t launch_gemv_ref_gather(int type, const void* w, int64_t N, int64_t K,
                                   uint16_t* y, float* y_f32, int nslots, const int32_t* sel, int topk, int64_t E,
                                   int64_t wstride, const void* w_alt, int64_t x_zstride, int64_t y_zstride,
                                   hipStream_t st, const void* w2, const void* w2_alt, uint16_t* y2) {
-    const uint8_t* W = (const uint8_t*)w;
     const RefGather ga{sel, topk, nslots, (const uint8_t*)w2, (const uint8_t*)w2_alt, y2, E, wstride,
                        (const uint8_t*)w_alt, x_zstride, y_zstride};
-    if (w2) nslots *= 2;
-    switch (type) {
-        case T_Q4_K: return run_ref_type<T_Q4_K>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-        case T_Q6_K: return run_ref_type<T_Q6_K>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-        case T_Q8_0: return run_ref_type<T_Q8_0>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-        case T_F16: return run_ref_type<T_F16>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-        case T_BF16: return run_ref_type<T_BF16>(W, N, K, x, M, y, y_f32, nslots, ga, st);
-        default: return hipErrorInvalidValue;
-    }
+    return run_ref_any(type, RefCall{(const uint8_t*)w, N, K, x, M, y, y_f32, N, w2 ? 2 * nslots : nslots, ga, st});
 }
 
 hipError_t launch_gemv_ref(int type, const void* w, int64_t N, int64_t K, const uint16_t* x, int64_t M,
@@ -614,13 +913,30 @@ hipError_t launch_gemv_ref(int type, const void* w, int64_t N, int64_t K, const 
 hipError_t launch_gemv_ref_tiles(const aipu_tile_desc* tiles, int n_tiles, int64_t K, const uint16_t* x, int64_t M,
                                  uint16_t* y, float* y_f32, int64_t ys, hipStream_t st) {
     if (n_tiles < 1 || n_tiles > AIPU_MAX_TILES || M < 1) return hipErrorInvalidValue;
+    // tiles of so many rows that the one-wave kernel is faster run by themselves, the others in one launch
+    aipu_tile_desc rest[AIPU_MAX_TILES];
+    int n_rest = 0;
+    for (int i = 0; i < n_tiles; ++i) {
+        const aipu_tile_desc& d = tiles[i];
+        const RefCall c{(const uint8_t*)d.w, d.nrows, K, x, M, y + d.row0, y_f32 ? y_f32 + d.row0 : nullptr, ys, 1, RefGather{}, st};
+        const int64_t mc = M >= 5 ? 8 : M >= 3 ? 4 : M;
+        if (!ref_wave_takes(d.ggml_type, c) || !ref_wave_wins(d.ggml_type, d.nrows * ((M + mc - 1) / mc), M, K)) {
+            rest[n_rest++] = d;
+            continue;
+        }
+        const hipError_t e = run_ref_any(d.ggml_type, c);
+        if (e != hipSuccess) return e;
+    }
+    if (n_rest == 0) return hipSuccess;
+    tiles = rest;
+    n_tiles = n_rest;
     int64_t rows = 0;
     for (int i = 0; i < n_tiles; ++i) rows += tiles[i].nrows;
     const auto run = [&](auto cfg, auto kernel, int mc, int rm) {
         typedef decltype(cfg) C;
         // a launch's threads must fit 32 bits: pieces of at most kMaxRows rows, flushed before they exceed it
         constexpr int64_t kMaxWgs = 0xFFFFFFFFLL / C::kThreads;
-        const int R = ref_rows_per_wg(rows, rm);
+        const int R = ref_rows_per_wg(rows * ((M + mc - 1) / mc), rm);
         RefTiles a{};
         int64_t nwg = 0;
         const auto flush = [&] {

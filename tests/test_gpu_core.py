@@ -231,6 +231,40 @@ def test_gemv_ref_row_split(t, N, K, M):
     assert_bits_equal(h_bits(y), ye, "y")
 
 
+# Many rows: one wave per 64 rows.  A ragged last wave, one and several chunks of 256 activations, a last
+# chunk of one unit (K = 320), both 2-byte phases of Q6_K blocks, every pass width, a leftover pass
+# (M = 9), 4 waves per CU (16 bits, M = 2, K = 2048), and pointers or K that stay on the producer kernel.
+WAVE_CASES = [
+    (qo.GGML_Q4_K, 40001, 256, 1), (qo.GGML_Q4_K, 25001, 768, 2), (qo.GGML_Q4_K, 50001, 512, 3), (qo.GGML_Q4_K, 37003, 256, 9),
+    (qo.GGML_Q6_K, 17001, 1024, 1), (qo.GGML_Q6_K, 17030, 512, 2), (qo.GGML_Q6_K, 34001, 512, 4), (qo.GGML_Q6_K, 17001, 768, 1),
+    (qo.GGML_Q8_0, 31001, 192, 1), (qo.GGML_Q8_0, 25002, 576, 2), (qo.GGML_Q8_0, 50001, 640, 4), (qo.GGML_Q8_0, 60001, 64, 8),
+    (qo.GGML_F16, 34001, 320, 1), (qo.GGML_F16, 113001, 2048, 2), (qo.GGML_F16, 34001, 448, 3), (30, 34001, 832, 1),
+    (30, 60001, 128, 8),
+]
+
+
+@pytest.mark.parametrize("t,N,K,M", WAVE_CASES)
+def test_gemv_ref_many_rows(t, N, K, M):
+    note(f"gemv ref many rows type={t} N={N} K={K} M={M}")
+    rng = np.random.default_rng(N + K + M)
+    x = qo.random_bf16(rng, (M, K))
+    few = 256   # rows of the oracle, repeated down the matrix
+    raw = qo.random_bf16(rng, few * K).view(np.uint8) if t == 30 else qo.random_weights(rng, t, few, K)
+    if t == 30:
+        acc, ye = qo.gemv_ref(qo.bf16_bits_to_f32(raw.view(np.uint16)).reshape(few, K), qo.bf16_bits_to_f32(x))
+    else:
+        acc, ye = co.gemv_ref(t, raw, few, K, x)
+    w = d_u8(raw).view(few, -1).repeat((N + few - 1) // few, 1)[:N].contiguous().view(-1)
+    reps = (N + few - 1) // few
+    for off in (0, 1):   # 8-byte aligned activations, and not
+        buf = torch.zeros(M * K + 8, dtype=torch.int16, device="cuda")
+        buf[off:off + M * K] = torch.from_numpy(x.reshape(-1).view(np.int16)).to("cuda")
+        xd = buf[off:off + M * K].view(torch.bfloat16).view(M, K)
+        y, yf = dev.gemv(t, w, N, K, xd, mode="ref", out_f32=True)
+        assert_bits_equal(u32(h_f32(yf)), np.tile(u32(acc), (1, reps))[:, :N], "acc")
+        assert_bits_equal(h_bits(y), np.tile(np.asarray(ye).reshape(M, few), (1, reps))[:, :N], "y")
+
+
 def test_gemv_ref_k_beyond_2_31():
     """A row of more than 2^31 weights: every offset into it and into the activations is 64-bit."""
     K, M = (1 << 31) + 48, 2

@@ -112,6 +112,20 @@ def test_moe_ref_bitexact(router_type, shared, topk):
     assert_bits_equal(h_bits(y), r["y"], "y")
 
 
+def test_moe_ref_many_rows():
+    """Gate and up of nine slots have so many rows that one wave per 64 rows takes them, both stacks
+    and the shared matrices in one launch."""
+    E, H, I, topk = 16, 256, 2048, 8
+    note("moe ref many rows")
+    rng = np.random.default_rng(88)
+    rw, ex, sh, x = _moe_case(rng, E, H, I, BF16, True)
+    y, sel, sw = dev.moe_swiglu_decode(BF16, d_u8(rw), Q4K, *map(d_u8, ex), E, H, I, topk, d_bf16(x), mode="ref",
+                                       shared=tuple(map(d_u8, sh)))
+    r = go.moe_decode_ref(x, BF16, rw, ex, Q4K, E, H, I, topk, shared=sh)
+    assert np.array_equal(sel.cpu().numpy(), r["sel_idx"])
+    assert_bits_equal(h_bits(y), r["y"], "y")
+
+
 @pytest.mark.parametrize("router_type,shared,topk", [(BF16, False, 4), (Q4K, True, 4), (Q4K, True, 8),
                                                     (BF16, True, 7)])
 def test_moe_fast_small(router_type, shared, topk):
@@ -646,6 +660,24 @@ def test_mixed_tiles_ref_one_launch(K, M, n_tiles, rows):
     assert np.all(gy[:, ~covered] == qo.bf16_round_bits(np.float32(7.0))), "rows outside the tiles written"
 
 
+def test_mixed_tiles_ref_long_tile():
+    """A tile of so many rows that it runs by itself, between short ones, with the output's row stride."""
+    K, M, n = 256, 2, 25000
+    note("tiles ref long tile")
+    rng = np.random.default_rng(29)
+    raw = [qo.random_weights(rng, t, r, K) for t, r in ((qo.GGML_Q8_0, 24), (Q4K, n), (qo.GGML_Q6_K, 40))]
+    x = qo.random_bf16(rng, (M, K))
+    N = n + 100
+    y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    rows = [(qo.GGML_Q8_0, 0, 24), (Q4K, 30, n), (qo.GGML_Q6_K, n + 40, 40)]
+    dev.gemv_tiles([(t, d_u8(w), r0, r) for w, (t, r0, r) in zip(raw, rows)], N, K, d_bf16(x), mode="ref", out=y)
+    got, covered = h_bits(y), np.zeros(N, bool)
+    for w, (t, r0, r) in zip(raw, rows):
+        assert_bits_equal(got[:, r0:r0 + r], np.asarray(co.gemv_ref(t, w, r, K, x)[1]).reshape(M, r), f"tile at {r0}")
+        covered[r0:r0 + r] = True
+    assert np.all(got[:, ~covered] == qo.bf16_round_bits(np.float32(7.0))), "rows outside the tiles written"
+
+
 def test_mixed_tiles_ref_beyond_one_grid():
     """Tiles whose workgroups' threads do not fit one grid (2^28 rows at five activation rows) run in
     several launches."""
@@ -659,9 +691,12 @@ def test_mixed_tiles_ref_beyond_one_grid():
         w[r * 144:(r + 8) * 144] = d_u8(raw[i * 8 * 144:(i + 1) * 8 * 144])
     tail = d_u8(raw[32 * 144:])
     x = qo.random_bf16(rng, (M, K))
+    xb = torch.zeros(M * K + 1, dtype=torch.int16, device="cuda")   # 2-byte aligned: the one-launch kernel
+    xb[1:] = torch.from_numpy(x.reshape(-1).view(np.int16)).to("cuda")
     N = n0 + 16
     y = torch.ones((M, N), dtype=torch.bfloat16, device="cuda")
-    dev.gemv_tiles([(Q4K, w, 0, n0), (Q4K, tail, n0, 16)], N, K, d_bf16(x), mode="ref", out=y)
+    dev.gemv_tiles([(Q4K, w, 0, n0), (Q4K, tail, n0, 16)], N, K, xb[1:].view(torch.bfloat16).view(M, K), mode="ref",
+                   out=y)
     _, ye = co.gemv_ref(Q4K, raw, 48, K, x)
     ye = np.asarray(ye).reshape(M, 48)
     for i, r in enumerate(at):
