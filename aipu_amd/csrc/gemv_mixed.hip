@@ -574,21 +574,47 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
     }
     __syncthreads();
     const int m = tid / kTR, rr = tid - m * kTR;
-    if (m < MR && m < M && rr < nvalid) {
-        float v = 0.f;
+    const bool live = m < MR && m < M && rr < nvalid;
+    float v = 0.f;
+    if (live) {
 #pragma unroll
         for (int k = 0; k < kMixW; ++k) v += red[(m * kMixW + k) * kTR + rr];
-        const int64_t row = T.row0 + r0 + rr;
-        if constexpr (TYPE == T_BF16) {
-            // an infinite weight meets the zeros of the other K-groups' operands: a NaN is formed again
-            // without them, so that only a NaN of the product itself stays one
-            if (v != v) {
-                const uint16_t* wv = (const uint16_t*)(T.w + (int64_t)(r0 + rr) * rb);
-                v = 0.f;
-                for (int k = 0; k < K; ++k)
-                    v = __builtin_fmaf(bf16_to_f32(X[(int64_t)m * K + k]), bf16_to_f32(wv[k]), v);
+    }
+    if constexpr (TYPE == T_BF16) {
+        // an infinite weight meets the zeros of the other K-groups' operands: a NaN is formed again
+        // without them, so that only a NaN of the product itself stays one.  Wave 0 holds every output
+        // and forms each with all lanes; a NaN activation leaves its whole row as it is after one pass
+        // (one thread per output walking K took 446 us at 2048 x 6144, M = 4; 11 so, 9 without a NaN).
+        uint64_t bad = __ballot(live && v != v);
+        while (bad) {
+            const int o = __ffsll((unsigned long long)bad) - 1;
+            const uint16_t* xo = X + (int64_t)(o / kTR) * K;
+            const uint16_t* wo = (const uint16_t*)(T.w + (int64_t)(r0 + o % kTR) * rb);
+            float f = 0.f;
+            bool xnan = false;
+            for (int k = 8 * lane; k < K; k += 8 * 64) {
+                const uint4 x4 = *(const uint4*)(xo + k), w4 = *(const uint4*)(wo + k);
+                const uint32_t xw[4] = {x4.x, x4.y, x4.z, x4.w}, ww[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float xl = bf16_to_f32(xw[e] & 0xFFFFu), xh = __uint_as_float(xw[e] & 0xFFFF0000u);
+                    xnan |= xl != xl || xh != xh;
+                    f = __builtin_fmaf(xl, bf16_to_f32(ww[e] & 0xFFFFu), f);
+                    f = __builtin_fmaf(xh, __uint_as_float(ww[e] & 0xFFFF0000u), f);
+                }
             }
+            if (__any(xnan)) {
+                bad &= ~(((1ull << kTR) - 1) << (o / kTR * kTR));
+                continue;
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) f += __shfl_xor(f, d, 64);
+            if (lane == o) v = f;
+            bad &= bad - 1;
         }
+    }
+    if (live) {
+        const int64_t row = T.row0 + r0 + rr;
         Y[(int64_t)m * ys + row] = (uint16_t)bf16_rne(v);
         if (Yf) Yf[(int64_t)m * ys + row] = v;
     }

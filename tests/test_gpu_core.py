@@ -512,6 +512,31 @@ def test_gemv_fast_bf16_infinities(N, K):
     assert ok, worst
 
 
+@pytest.mark.parametrize("N,K,M", [(70, 256, 4), (70, 2560, 3), (2100, 3072, 4)])
+def test_gemv_fast_bf16_nan_rows(N, K, M):
+    """A NaN activation makes its row's outputs NaN and no others; a NaN weight its output of every row;
+    infinite weights beside them keep the other outputs' infinities."""
+    note(f"gemv fast bf16 NaN rows N={N} K={K} M={M}")
+    rng = np.random.default_rng(N + K + M)
+    w = qo.bf16_bits_to_f32(qo.random_bf16(rng, (N, K), scale=0.05))
+    x = qo.bf16_bits_to_f32(qo.random_bf16(rng, (M, K)))
+    x[x == 0] = 1.0
+    x[1, K - 3] = np.nan
+    w[5, K // 2], w[9, 7], w[20, 0], w[N - 1, K - 1] = np.nan, np.inf, -np.inf, np.inf
+    bits = (w.view(np.uint32) >> 16).astype(np.uint16)
+    xb = (x.view(np.uint32) >> 16).astype(np.uint16)
+    _, yf = _fast_rows(go.BF16_TYPE, d_u8(bits.reshape(-1).view(np.uint8)), N, K, xb, "fast")
+    got = yf.view(np.float32)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32)) and np.array_equal(np.isinf(got), inf)
+    fin = np.isfinite(want[0])
+    ok, worst = qo.tolerance_gate(w[fin], x[:1], got[:1, fin])
+    assert ok, worst
+
+
 # AIPU_MODE_FAST_DENSE: Q4_K batches of 2..8 rows at K = 2048/4096/6144 run the dense
 # multi-row kernel.  A row agrees with its one-row call within the fast-mode tolerance (fp32
 # gate, bf16 within 1 ulp where well conditioned), and its bits depend neither on the other
