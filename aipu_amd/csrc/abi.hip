@@ -81,8 +81,8 @@ int check_gemv(int type, const void* w, int64_t N, int64_t K, const void* x, int
     return AIPU_OK;
 }
 
-// Fast kernels exist for every type: Q4_K on the matrix cores, bf16 in the streaming
-// kernel, Q6_K / Q8_0 / F16 in the mixed-type kernel (K up to its staging limit).  Larger K,
+// Fast kernels exist for every type: Q4_K on the matrix cores, bf16 in the mixed-type kernel or the
+// streaming kernel by N and K, Q6_K / Q8_0 / F16 in the mixed-type kernel (K up to its staging limit).  Larger K,
 // and K that is not a whole number of 256-weight super-blocks, are served by the exact
 // kernel, whose results trivially satisfy the fast-mode tolerance.
 bool has_fast(int type, int64_t K) {

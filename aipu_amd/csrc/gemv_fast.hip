@@ -717,10 +717,12 @@ hipError_t launch_gemv_fast(int type, const void* w, int64_t N, int64_t K, const
         case T_BF16:
             // The matrix cores where one row is no slower there than in the streaming kernel, whose VALU
             // multiplies every row separately (the choice depends on N and K alone, so that the rows of a
-            // batch keep their one-row bits).  M = 1, streaming > matrix cores: K = 2048, N = 64 / 2048
-            // 4.7 > 3.6 / 5.7 > 4.7 us; K = 6144, N = 256 / 2048 / 8192 7.3 > 7.7 / 10.7 > 9.8 / 34 > 21;
-            // K = 8192, N = 512 / 8192 5.8 > 10.6 / 41 > 35.  M = 4 at 6144 x 6144: 86 > 17 us.
-            if (!(K <= 2560 || (K <= 6144 && N >= 2048)) || N > kMixedMaxN || !gemv_mixed_supported(type, K))
+            // batch keep their one-row bits).  M = 1, streaming > matrix cores: K = 2560, N = 16 / 1024 / 2048
+            // 4.4 > 4.0 / 4.6 > 4.6 / 4.7 > 4.6 us; K = 3072, N = 1024 4.6 > 4.6; K = 4096, N = 256 / 1024 / 1536 /
+            // 2048 / 2560 4.7 > 5.0 / 4.7 > 5.0 / 4.9 > 5.1 / 5.7 > 5.7 / 8.5 > 6.1; K = 6144, N = 256 / 2048 / 8192 6.0 >
+            // 6.3 / 8.1 > 6.6 / 34 > 21.  Beyond K = 6144 the matrix-core kernel takes two rows a pass and spills:
+            // K = 8192, N = 512 / 8192 5.8 > 10.6 / 41 > 35.  M = 4 at 6144 x 6144: 80 > 15 us.
+            if (!(K <= 3072 || (K <= 6144 && N > 1536)) || N > kMixedMaxN || !gemv_mixed_supported(type, K))
                 return gemv_stream_mc<T_BF16, 2>((const uint8_t*)w, N, K, x, M, y, y_f32, st);
             [[fallthrough]];
         case T_Q6_K:

@@ -48,6 +48,8 @@ namespace {
 constexpr int kMixW = 4;                  // waves per workgroup (= K parts)
 static_assert(kMixedMaxN / kTR * kMixW * 64 <= 0xFFFFFFFFLL, "a grid's threads along x fit 32 bits");
 constexpr int kSliceBytes = 9 * 1024;     // per-wave weight slice: the largest group below
+constexpr int kDeep = 3;                  // k_bf16_deep: slices per wave (four: 5.9 -> 6.3 us, 16 x 6144), their pitch
+constexpr int kDeepPitch = 8 * 1024;
 
 // Bytes of one 256-weight block of one row in memory (kBlk) and in the LDS slice (kPitch),
 // and blocks per streamed group (GS) of 16 rows.  A Q6_K block is copied as 14 whole 16-B
@@ -317,9 +319,34 @@ struct ActRegion {
     static constexpr int kSumOff = kRing * 512;
 };
 
-template <int TYPE, int XI, int MR>
+// The lane's 64 F16 / BF16 weights of a block from LDS, read and waited for inside one asm statement: the
+// compiler would order loads it can see behind every direct-to-LDS copy in flight.
+__device__ __forceinline__ Raw128 read128_lds(uint32_t a) {
+    u32x4_t v[8];
+    asm volatile(
+        "ds_read_b128 %0, %8\n\t"
+        "ds_read_b128 %1, %8 offset:16\n\t"
+        "ds_read_b128 %2, %8 offset:32\n\t"
+        "ds_read_b128 %3, %8 offset:48\n\t"
+        "ds_read_b128 %4, %8 offset:64\n\t"
+        "ds_read_b128 %5, %8 offset:80\n\t"
+        "ds_read_b128 %6, %8 offset:96\n\t"
+        "ds_read_b128 %7, %8 offset:112\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+        : "v"(a)
+        : "memory");
+    Raw128 r;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) r.v[s] = make_uint4(v[s].x, v[s].y, v[s].z, v[s].w);
+    return r;
+}
+
+// DEPTH: groups in flight per wave, each in a slice of its own (more than one: 16-bit types only).
+// RG: rows per workgroup, at most 16 (a row's result does not depend on it).
+template <int TYPE, int XI, int MR, int DEPTH = 1>
 __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16_t* __restrict__ X, int K, int M,
-                                         uint8_t* wA, uint8_t* wW, float* red, uint16_t* Y, float* Yf, int64_t ys) {
+                                         uint8_t* wA, uint8_t* wW, float* red, uint16_t* Y, float* Yf, int64_t ys, int RG = kTR) {
     typedef Geom<TYPE> G;
     typedef ActRegion AR;
     static_assert(G::GS <= 3, "a group must not reach back to the slots it restages");
@@ -331,8 +358,8 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
     const int bpk = kb1 - kb0;
     const int NG = (bpk + G::GS - 1) / G::GS;
     const int64_t rb = (int64_t)nsb * G::kBlk;
-    const int r0 = grp * kTR;
-    const int nvalid = T.nrows - r0 < kTR ? T.nrows - r0 : kTR;
+    const int r0 = grp * RG;
+    const int nvalid = T.nrows - r0 < RG ? T.nrows - r0 : RG;
 
     // 1. this wave's activations of every row (pieces past its blocks, and rows past M, read
     // as zero), 2. its first group
@@ -351,6 +378,8 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
     MixDma<TYPE> dma;
     dma.init(lane, rb);
     dma.issue(wr, wW, kb0, bpk < G::GS ? bpk : G::GS);
+#pragma unroll
+    for (int d = 1; d < DEPTH; ++d) dma.issue(wr, wW + d * kDeepPitch, kb0 + d * G::GS, bpk - d * G::GS);
     __builtin_amdgcn_sched_barrier(0);
 
     // 3. the row exponents (fp16 operands), then stage blocks 0..3 (every piece, so blocks past
@@ -520,14 +549,21 @@ __device__ __forceinline__ void mix_body(const MixTile& T, int grp, const uint16
         f32x4_t D0 = {0.f, 0.f, 0.f, 0.f}, D1 = {0.f, 0.f, 0.f, 0.f};
         float acc1[MR] = {}, p0[MR] = {}, p1[MR] = {};
         for (int gi = 0; gi < NG; ++gi) {
-            __builtin_amdgcn_s_waitcnt(kWaitVm0);
-            const uint8_t* p = wW + rrow + 128 * g;
+            // the later groups' copies (zeros past the part) stay in flight
+            __builtin_amdgcn_s_waitcnt(DEPTH == 1 ? kWaitVm0 : wait_vm((DEPTH - 1) * MixDma<TYPE>::kInsts));
+            uint8_t* const slice = wW + (DEPTH == 1 ? 0 : gi % DEPTH) * kDeepPitch;
             Raw128 R[1];
+            if constexpr (DEPTH == 1) {
+                const uint8_t* p = slice + rrow + 128 * g;
 #pragma unroll
-            for (int s = 0; s < 8; ++s) R[0].v[s] = *(const uint4*)(p + 16 * s);
-            if (gi + 1 < NG) {
-                regs_consumed(R);   // the slice has been read: refill it
-                dma.issue(wr, wW, kb0 + gi + 1, bpk - gi - 1);
+                for (int s = 0; s < 8; ++s) R[0].v[s] = *(const uint4*)(p + 16 * s);
+                if (gi + 1 < NG) {
+                    regs_consumed(R);   // the slice has been read: refill it
+                    dma.issue(wr, slice, kb0 + gi + 1, bpk - gi - 1);
+                }
+            } else {
+                R[0] = read128_lds(lds_addr(slice) + rrow + 128u * (uint32_t)g);
+                dma.issue(wr, slice, kb0 + gi + DEPTH, bpk - gi - DEPTH);
             }
             restage(gi);
             a_reads(A, aLane + 512u * (uint32_t)slot(gi), dmask);
@@ -648,6 +684,22 @@ __global__ __launch_bounds__(kMixW * 64) void k_mixed(MixArgs args, const uint16
     }
 }
 
+// A plain bf16 GEMV of few rows: `rg` rows per workgroup, so that as many CUs as possible have one, and
+// several groups in flight per wave, which take the LDS that a second workgroup would.  With 16 rows and
+// one group in flight 2048 x 3584 took 6.1 us at M = 1, more than the streaming kernel's 4.8.
+template <int XI, int MR>
+__global__ __launch_bounds__(kMixW * 64) void k_bf16_deep(MixTile T, const uint16_t* __restrict__ X, int K, int M,
+                                                          uint16_t* __restrict__ Y, float* __restrict__ Yf, int64_t ys, int rg) {
+    typedef ActRegion AR;
+    static_assert(MixDma<T_BF16>::kInsts * 1024 <= kDeepPitch, "slice too small");
+    __shared__ __align__(16) uint8_t s_act[kMixW * MR * AR::kBytes];
+    __shared__ float red[MR * kMixW * kTR];
+    extern __shared__ __align__(16) uint8_t s_w[];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    mix_body<T_BF16, XI, MR, kDeep>(T, (int)blockIdx.x, X, K, M, s_act + w * MR * AR::kBytes,
+                                              s_w + w * kDeep * kDeepPitch, red, Y, Yf, ys, rg);
+}
+
 // Blocks per wave that k_mixed<XI> loads as XI 16-B pieces per lane and row (every type's groups
 // rounded up to whole groups must fit): 2 XI blocks.  A wave's bpk blocks round up to
 // max(3 ceil(bpk / 3), 2 ceil(bpk / 2)) = 3, 3, 4, 6, 6, 6, 9, 9, ... blocks, so 1-3 blocks per
@@ -708,6 +760,10 @@ hipError_t launch_gemv_mixed(const aipu_tile_desc* tiles, int n_tiles, int64_t K
     const dim3 grid((unsigned)nwg), block(kMixW * 64);
     const size_t lds = (size_t)kMixW * kSliceBytes;
     const int xi = mix_xi(K), mrmax = mix_rows(xi);
+    const bool deep = n_tiles == 1 && tiles[0].ggml_type == T_BF16 && xi <= 3 && nwg <= device_cu_count();
+    // k_bf16_deep: rows per workgroup (four were slower again, 1024 x 2560 5.0 against 4.6 us)
+    const int rg = (tiles[0].nrows + 7) / 8 <= device_cu_count() ? 8 : kTR;
+    const dim3 dgrid((unsigned)((tiles[0].nrows + rg - 1) / rg));
     for (int64_t m0 = 0; m0 < M;) {
         const int rows = (int)(M - m0 < mrmax ? M - m0 : mrmax);
         const uint16_t* xm = x + m0 * K;
@@ -716,10 +772,20 @@ hipError_t launch_gemv_mixed(const aipu_tile_desc* tiles, int n_tiles, int64_t K
         const int mr = rows > 2 ? 4 : rows;
 #define AIPU_MIX(XV, MV) \
     if (xi == XV && mr == MV) hipLaunchKernelGGL((k_mixed<XV, MV>), grid, block, lds, st, a, xm, (int)K, rows, ym, yfm, ys);
-        AIPU_MIX(2, 1) AIPU_MIX(2, 2) AIPU_MIX(2, 4)
-        AIPU_MIX(3, 1) AIPU_MIX(3, 2) AIPU_MIX(3, 4)
-        AIPU_MIX(8, 1) AIPU_MIX(8, 2)
+#define AIPU_DEEP(XV, MV)                                                                                                   \
+    if (xi == XV && mr == MV)                                                                                               \
+        hipLaunchKernelGGL((k_bf16_deep<XV, MV>), dgrid, block, kMixW * kDeep * kDeepPitch, st, a.t[0], xm,         \
+                           (int)K, rows, ym, yfm, ys, rg);
+        if (deep) {
+            AIPU_DEEP(2, 1) AIPU_DEEP(2, 2) AIPU_DEEP(2, 4)
+            AIPU_DEEP(3, 1) AIPU_DEEP(3, 2) AIPU_DEEP(3, 4)
+        } else {
+            AIPU_MIX(2, 1) AIPU_MIX(2, 2) AIPU_MIX(2, 4)
+            AIPU_MIX(3, 1) AIPU_MIX(3, 2) AIPU_MIX(3, 4)
+            AIPU_MIX(8, 1) AIPU_MIX(8, 2)
+        }
 #undef AIPU_MIX
+#undef AIPU_DEEP
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         m0 += rows;

@@ -469,9 +469,12 @@ def test_gemv_fast_batch_invariance_bf16(N, K, M):
         assert_bits_equal(y1[0], yb[r], f"bf16 row {r} of M={M}: bf16 outputs")
 
 
-# bf16 weights take the matrix cores up to K = 2560, and up to K = 6144 from 2048 rows on, else the
-# streaming kernel: both sides of each line, ragged row groups, batches in passes of four.
-@pytest.mark.parametrize("N,K,M", [(33, 2560, 1), (2047, 2816, 2), (2049, 2816, 3), (2050, 6144, 5), (70, 6400, 4), (15, 256, 8)])
+# bf16 weights take the matrix cores up to K = 3072, and up to K = 6144 beyond 1536 rows, else the
+# streaming kernel: both sides of each line, eight and sixteen rows per workgroup (2048 rows on 256 CUs),
+# one and several workgroups per CU (4096), ragged row groups, fewer blocks than waves, the copies'
+# ring of three slices full, not full and passed twice, batches in passes of four.
+@pytest.mark.parametrize("N,K,M", [(33, 2560, 1), (2047, 2816, 2), (2049, 2816, 3), (2050, 6144, 5), (70, 6400, 4), (15, 256, 8),
+                                   (1536, 3328, 2), (1537, 3328, 4), (9, 3072, 3), (2047, 6144, 2), (4095, 3584, 4), (4100, 2304, 2)])
 def test_gemv_fast_bf16_dispatch(N, K, M):
     note(f"gemv fast bf16 dispatch N={N} K={K} M={M}")
     rng = np.random.default_rng(19 * N + K + M)
