@@ -1191,7 +1191,9 @@ hipError_t launch_gemv_mfma(const void* w, int64_t N, int64_t K, const uint16_t*
         uint16_t* ym = y + m0 * ystride;
         float* yfm = y_f32 ? y_f32 + m0 * ystride : nullptr;
         if (left >= 2 && canon1) {
-            if (left == 2 && !dense && gemv_persist2_supported(N, K)) {   // two rows on the one-row kernel
+            // two rows on the one-row kernel (dense: where neither the dense kernel nor k_gemvs serves the
+            // shape; 512 x 4352 3.8 us there and 4.4 on the any-K kernel)
+            if (left == 2 && gemv_persist2_supported(N, K) && (!dense || (!small && !gemv_persist_m_supported(N, K, 2, true)))) {
                 const hipError_t e = launch_gemv_persist2(W, N, K, xm, ym, yfm, ystride, st);
                 if (e != hipSuccess) return e;
                 m0 += 2;

@@ -426,6 +426,22 @@ def test_gemv_fast_any_k_rows(N, K, M):
     assert ok, f"batch of M={M}: fp32 accumulators {worst:.3f} of the tolerance"
 
 
+@pytest.mark.parametrize("N,K,M", [(512, 4352, 2), (100, 2816, 2), (6144, 2816, 10), (16384, 4352, 2)])
+def test_gemv_dense_two_rows_without_dense_kernel(N, K, M):
+    """Dense mode at block counts without a dense kernel: two rows (or two left of a batch) on the one-row
+    kernel or the any-K kernel, every row with its one-row bits."""
+    note(f"gemv dense two rows N={N} K={K} M={M}")
+    rng = np.random.default_rng(N + K + M)
+    raw = qo.random_q4k_blocks(rng, N * K // 256)
+    x = qo.random_bf16(rng, (M, K))
+    wd = d_u8(raw)
+    yb, yfb = _fast_rows(qo.GGML_Q4_K, wd, N, K, x, "fast_dense")
+    for r in range(M):
+        y1, yf1 = _fast_rows(qo.GGML_Q4_K, wd, N, K, x[r:r + 1], "fast")
+        assert_bits_equal(yf1[0], yfb[r], f"row {r}: fp32 accumulators")
+        assert_bits_equal(y1[0], yb[r], f"row {r}: bf16 outputs")
+
+
 def _random_fast_cases(n=20, seed=1202):
     """Seeded Q4_K shapes for the fast mode's kernel choice: N from one tile to many per CU, K from
     one block to 8192 (one- and two-pair persistent waves, odd block counts), M = 1..8."""
