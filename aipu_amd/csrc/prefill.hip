@@ -645,13 +645,15 @@ __global__ __launch_bounds__(kSplitW * 64) __attribute__((amdgpu_waves_per_eu(R 
 // The smallest tile (the shortest walk per super-block) that leaves every
 // CU at most one workgroup, and no larger than M needs; up to six workgroups per CU in all.  Measured
 // at K = 6144, 128 x 256 kernel > split (M x N): 16 x 6144 108 > 18 us, 64 x 2048 112 > 19, 64 x 6144
-// 112 > 25, 100 x 6144 117 > 36, 256 x 6144 118 > 57, 512 x 6144 119 > 95, 128 x 16384 121 > 68;
-// beyond, 256 x 16384 123 and 123, 512 x 16384 133 against 237.
-int split_tile(int64_t M, int64_t N) {
+// 112 > 25, 100 x 6144 114 > 31, 256 x 6144 118 > 57, 512 x 6144 119 > 95, 128 x 16384 121 > 68;
+// beyond, 256 x 16384 123 and 123, 512 x 16384 133 against 237.  The limit holds at K = 512 .. 12288 (64
+// points each): both kernels' times follow K.  One super-block leaves seven of the eight waves
+// nothing to do: up to four workgroups per CU there (512 x 4096 21 > 19 us; 512 x 6144 22 and 27).
+int split_tile(int64_t M, int64_t N, int64_t K) {
     const int64_t nt = (N + 31) / 32, cus = device_cu_count();
     const auto wgs = [&](int ms) { return (M + 16 * ms - 1) / (16 * ms) * nt; };
     const int ms = M <= 16 || wgs(1) <= cus ? 1 : M <= 32 || wgs(2) <= cus ? 2 : 4;
-    return wgs(ms) <= 6 * cus ? ms : 0;
+    return wgs(ms) <= (K == QK_K ? 4 : 6) * cus ? ms : 0;
 }
 
 int64_t mpad(int64_t M) { return (M + kBM - 1) / kBM * kBM; }
@@ -673,7 +675,7 @@ hipError_t launch_gemm_prefill(int type, const void* w, int64_t N, int64_t K, co
     if ((int64_t)mtiles * ntiles > 0x7FFFFFFF || (int64_t)64 * nsb * 144 >= (1LL << 32)) return hipErrorInvalidValue;
     uint8_t* chunks = (uint8_t*)ws;
     int32_t* rexp = (int32_t*)(chunks + (int64_t)mtiles * nsb * kChunk);
-    const int ms = split_tile(M, N);   // 16-row subtiles of the split kernel's tile, 0: the 128 x 256 kernel
+    const int ms = split_tile(M, N, K);   // 16-row subtiles of the split kernel's tile, 0: the 128 x 256 kernel
     // rows staged: what the GEMM reads
     const int64_t Ms = ms ? (M + 16 * ms - 1) / (16 * ms) * (16 * ms) : Mp;
     if (K <= kStageMaxK) {

@@ -55,8 +55,9 @@ def test_prefill_tolerance_shapes(M, N, K):
 
 # The split kernel's tiles (16, 32 and 64 rows; 64 with one and with more workgroups per CU) at ragged M
 # and N, fewer super-blocks than waves and uneven parts; and the 128 x 256 kernel ragged on both sides.
+# One super-block: up to four workgroups per CU (400 x 4100), beyond on the 128 x 256 kernel (300 x 8000).
 SPLIT_CASES = [(16, 6001, 512), (1, 33, 256), (17, 4200, 512), (40, 4100, 256), (33, 8200, 512), (32, 16400, 256),
-               (300, 40, 2304), (5, 24, 1792), (130, 16400, 256)]
+               (300, 40, 2304), (5, 24, 1792), (130, 16400, 256), (400, 4100, 256), (300, 8000, 256)]
 
 
 @pytest.mark.parametrize("M,N,K", SPLIT_CASES)
