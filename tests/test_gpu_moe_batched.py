@@ -206,11 +206,12 @@ def test_batched_fast_two_row_pass_equals_one_row_pass(H, topk, shared):
     _check_fast(y2, sel2, sw2, X[:2], BF16, rw, ex, sh, E, H, I, topk)
 
 
-@pytest.mark.parametrize("M,E,topk,shared", [(7, 8, 8, True), (8, 4, 4, False), (9, 3, 2, True), (8, 600, 8, True)])
+@pytest.mark.parametrize("M,E,topk,shared", [(7, 8, 8, True), (8, 4, 4, False), (9, 3, 2, True), (8, 600, 8, True),
+                                                (5, 40, 32, True), (2, 33, 17, False), (3, 16, 9, True)])
 def test_batched_fast_slot_lists(M, E, topk, shared):
     """The slot lists of a pass at their limits: every row on every expert (four slots each, the
-    last one half empty at seven rows), fewer experts than rows, a leftover row, and routing outside
-    the one-workgroup kernel; within the fast-mode bound, and every row equal to a two-row batch."""
+    last one half empty at seven rows), fewer experts than rows, a leftover row, routing outside
+    the one-workgroup kernel, and more than eight and sixteen experts per row; within the fast-mode bound, and every row equal to a two-row batch."""
     H, I = 512, 256
     note(f"moe batched fast slot lists M={M} E={E} topk={topk} shared={shared}")
     rng = np.random.default_rng(31 * M + E)
