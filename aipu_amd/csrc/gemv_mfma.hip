@@ -1192,7 +1192,7 @@ hipError_t launch_gemv_mfma(const void* w, int64_t N, int64_t K, const uint16_t*
         float* yfm = y_f32 ? y_f32 + m0 * ystride : nullptr;
         if (left >= 2 && canon1) {
             // two rows on the one-row kernel (dense: where neither the dense kernel nor k_gemvs serves the
-            // shape; 512 x 4352 3.8 us there and 4.4 on the any-K kernel)
+            // shape; 512 x 4352 3.8 us there and 4.4 on k_gemvr)
             if (left == 2 && gemv_persist2_supported(N, K) && (!dense || (!small && !gemv_persist_m_supported(N, K, 2, true)))) {
                 const hipError_t e = launch_gemv_persist2(W, N, K, xm, ym, yfm, ystride, st);
                 if (e != hipSuccess) return e;
@@ -1205,8 +1205,9 @@ hipError_t launch_gemv_mfma(const void* w, int64_t N, int64_t K, const uint16_t*
                 m0 += left;
                 continue;
             }
-            // the any-K kernel: beyond K = 6144, and where no kernel that holds a wave's whole part has
-            // a plan (two rows of those go to the one-row kernel above where it serves them)
+            // k_gemvr: beyond K = 6144 (five to eight rows at K = 8192: 21.1 us on k_gemvm, 17.5 there), and
+            // where no kernel that holds a wave's whole part has a plan (two rows of those go to the
+            // one-row kernel above where it serves them)
             if ((K > 6144 || !(left >= 5 ? gemvm_supported(nsb, 8) : small)) && gemv_rows_supported(N, K, left)) {
                 const hipError_t e = launch_gemv_rows(W, N, K, xm, left, ym, yfm, ystride, st);
                 if (e != hipSuccess) return e;

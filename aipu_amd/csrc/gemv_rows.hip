@@ -1,10 +1,11 @@
-// Multi-row Q4_K GEMV for any K (tolerance mode, M = 2 .. 8 activation rows, one weight pass),
-// in the one-row order of mfma_gemv.hpp: every row is bit-identical to its one-row launch.
+// Multi-row Q4_K GEMV for long or unevenly divided K (tolerance mode, M = 2 .. 8 activation rows, one
+// weight pass), in the one-row order of mfma_gemv.hpp: every row is bit-identical to its one-row launch.
 //
-// It serves the shapes the persistent multi-row kernels and the register-resident small-batch
-// kernel do not (they hold a wave's whole part of K): long K and block counts that do not split
-// into at most eight parts of three.  There a batch used to run one launch per row, reading the
-// weights M times.
+// It serves 8 .. 64 blocks where the persistent multi-row kernels and the register-resident small-batch
+// kernels (which hold a wave's whole part of K) have no plan and a one-row kernel forms the same order: up
+// to K = 8192 the block counts that do not split into at most eight parts of three (2816, 4352, 5632) and
+// every K beyond 6144; beyond 8192 those that k_gemv1 splits into at most eight parts of eight (8960, 9216,
+// 10240, 10752, 12288, .., 16384).  Any other K beyond 8192 runs a launch per row, or the streaming kernel.
 //
 // A workgroup owns a 16-row tile, wave w the w-th part of its blocks.  A wave walks its part block by
 // block with kNS blocks in flight: a block's weights arrive in one of its kNS LDS slots by
@@ -259,23 +260,21 @@ int64_t rows_lds(int nsb, int w) {
     return (int64_t)w * (MR * kActRow) + (int64_t)nsb * term_stride<MR>() * 4;   // dynamic
 }
 
-// Waves per workgroup: the most (up to eight, no more than blocks) that leave two workgroups on a
-// CU, unless that is under four; else the most that fit one; 0 if not even one wave does.
+constexpr int kMinBlocks = kRowMaxW, kMaxBlocks = 64;
+static_assert(kRowMaxW * 8 * kActRow + kMaxBlocks * term_stride<8>() * 4 <= 160 * 1024 - kRowMaxW * kNS * kSlot, "LDS");
+
+// Waves per workgroup: the most that leave two workgroups on a CU, unless that is under four; else eight.
 template <int MR>
 int rows_waves(int nsb) {
-    const int most = nsb < kRowMaxW ? nsb : kRowMaxW;
-    for (int w = most; w >= 4 || (w == most && w >= 1); --w)
+    for (int w = kRowMaxW; w >= 4; --w)
         if (rows_lds<MR>(nsb, w) <= 80 * 1024 - kRowMaxW * kNS * kSlot) return w;
-    for (int w = most; w >= 1; --w)
-        if (rows_lds<MR>(nsb, w) <= 160 * 1024 - kRowMaxW * kNS * kSlot) return w;
-    return 0;
+    return kRowMaxW;
 }
 
 template <int MR>
 hipError_t run_rows_any(const uint8_t* W, int64_t N, int nsb, const uint16_t* x, int M, uint16_t* y, float* yf, int64_t ys,
                         hipStream_t st) {
     const int w = rows_waves<MR>(nsb);
-    if (w == 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gemvr<MR>, dim3((unsigned)((N + kTR - 1) / kTR)), dim3(64 * w), (size_t)rows_lds<MR>(nsb, w), st, W, N,
                        nsb, x, M, y, yf, ys);
     return hipGetLastError();
@@ -284,9 +283,7 @@ hipError_t run_rows_any(const uint8_t* W, int64_t N, int nsb, const uint16_t* x,
 }  // namespace
 
 bool gemv_rows_supported(int64_t N, int64_t K, int M) {
-    if (M < 2 || M > 8 || N < 1 || N > kMaxN || K < QK_K || K % QK_K != 0 || K > (1 << 20)) return false;
-    const int nsb = (int)(K / QK_K);
-    return (M <= 2 ? rows_waves<2>(nsb) : M <= 4 ? rows_waves<4>(nsb) : rows_waves<8>(nsb)) > 0;
+    return M >= 2 && M <= 8 && N >= 1 && N <= kMaxN && K % QK_K == 0 && K >= kMinBlocks * QK_K && K <= kMaxBlocks * QK_K;
 }
 
 hipError_t launch_gemv_rows(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int M, uint16_t* y, float* yf,

@@ -91,8 +91,8 @@ hipError_t wait_gave_up_gemv_persist(uint32_t* flag);
 hipError_t wait_gave_up_gemv_persist_m(uint32_t* flag);
 hipError_t wait_gave_up_moe_persist(uint32_t* flag);
 
-// gemv_rows.hip -- Q4_K GEMV of 2 .. 8 activation rows at any K, one weight pass (tolerance mode,
-// each row bit-identical to the single-row kernels)
+// gemv_rows.hip -- Q4_K GEMV of 2 .. 8 activation rows at K = 2048 .. 16384, whatever K divides into, one
+// weight pass (tolerance mode, each row in the order of the single-row kernels of mfma_gemv.hpp)
 bool gemv_rows_supported(int64_t N, int64_t K, int M);
 hipError_t launch_gemv_rows(const uint8_t* W, int64_t N, int64_t K, const uint16_t* x, int M, uint16_t* y, float* yf,
                             int64_t ys, hipStream_t st);

@@ -102,7 +102,7 @@ def test_fp32_rsqrt_golden():
 
 
 # ------------------------------------------------------- reference-order GEMV
-# One kernel serves every type and K: passes of eight activation rows at most (9 rows at K = 256:
+# One kernel serves these types and K (many rows: WAVE_CASES): passes of eight activation rows at most (9 rows at K = 256:
 # 8 + 1), Q6_K blocks alternately 4-B aligned and 2 B past a dword, long K (32768, 40960).
 # Ragged N leaves part of the last wave idle.
 REF_CASES = [
@@ -132,7 +132,7 @@ def test_gemv_ref_bitexact(t, N, K, M):
 @pytest.mark.parametrize("t", [qo.GGML_Q4_K, qo.GGML_Q6_K, qo.GGML_Q8_0, qo.GGML_F16])
 def test_gemv_ref_unaligned_activations(t):
     """Reference mode asks only 2-byte aligned activations (and, below Q4_K, weights): a vector
-    that starts one element into its buffer takes the staged-weights kernel and stays bit-exact."""
+    that starts one element into its buffer stays bit-exact."""
     N, K, M = 96, 1024, 2
     note(f"gemv ref unaligned activations type={t}")
     rng = np.random.default_rng(4242 + t)
@@ -149,8 +149,8 @@ def test_gemv_ref_unaligned_activations(t):
 
 
 def _random_ref_cases(n=24, seed=20261202):
-    """Seeded shapes for the reference-order kernels: every type, ragged N, M = 1..9, K at the
-    register kernels' multiples (Q4_K 256, Q6_K 512, Q8_0 / F16 / BF16 64) and off them."""
+    """Seeded shapes for the reference order: every type, ragged N, M = 1..9, K a multiple of the
+    blocks of several types (256, 512, 64) and off them."""
     rng = np.random.default_rng(seed)
     kinds = [(qo.GGML_Q4_K, 256), (qo.GGML_Q6_K, 256), (qo.GGML_Q8_0, 32), (qo.GGML_F16, 1), (30, 1)]
     cases = []
@@ -350,11 +350,10 @@ def test_gemv_fast_tolerance(N, K, M):
 # PE_M = 1 runs (Makefile:1488-1508), and speculative decoding "changes speed, never output"
 # (PROJECT_BRIEFING.md:50).  In fast mode every row of an M-row call is bit-identical to the
 # one-row call on that row, fp32 accumulators included: the persistent row-pair kernel
-# (M = 2..8 at K = 2048/4096/6144), k_gemvs / k_gemvm elsewhere, and a launch per row where no
-# multi-row kernel forms rows in the one-row order (K / 256 not split into at most 8 parts of
-# at most 4 blocks: 2816, 5632; M = 1 off the persistent kernel: K > 8192), and the streaming
-# kernel beyond the matrix-core staging limit.  Two rows share a persistent launch wherever
-# nothing else takes them (odd prime block counts such as 23).
+# (M = 2..8 at K = 2048/4096/6144), k_gemvs / k_gemvm elsewhere up to K = 6144, k_gemvr at block counts
+# those do not split (2816, 5632) and at longer K, a launch per row or the streaming kernel where no
+# one-row kernel forms k_gemvr's order (some K > 8192), and the streaming kernel beyond the
+# matrix-core staging limit.  Two rows share a persistent launch up to K = 6144.
 # Covers every row count of a verify batch at the BASELINE shape, the other matrix-core shapes
 # (ragged N, passes of 8 + remainder), the shapes without a multi-row kernel, and K > 8192.
 INVARIANCE_CASES = [(6144, 6144, m) for m in (2, 3, 4, 5, 6, 7, 8)] + [
@@ -365,7 +364,7 @@ INVARIANCE_CASES = [(6144, 6144, m) for m in (2, 3, 4, 5, 6, 7, 8)] + [
     # one-row calls on the 16-row-tile kernel (k_gemv1) against batches on the row-pair and
     # small-batch kernels
     (4096, 2048, 3), (8192, 4096, 2), (4096, 8192, 2),
-    # no multi-row kernel in the one-row order: one launch per row
+    # block counts without a plan of the small-batch kernels: k_gemvr (two rows: the one-row kernel)
     (300, 2816, 5), (64, 5632, 2),
     # K > 8192: the one-row kernel is k_gemv1 (several weight-copy rounds); beyond the
     # matrix-core staging limit (K > 30464) every M runs the streaming kernel
@@ -375,8 +374,8 @@ INVARIANCE_CASES = [(6144, 6144, m) for m in (2, 3, 4, 5, 6, 7, 8)] + [
     # for it, a single block
     (100, 2304, 2), (6100, 6144, 2), (8192, 6144, 2), (8200, 4096, 2), (1, 256, 2),
     # block counts that no k_mfma_gemv plan splits (17, 19, 23, 29, 31 blocks): one-row calls on
-    # the persistent kernel, batches two rows at a time on it (K <= 6144) or a launch per row;
-    # and 37 blocks (K > 8192), where every M runs the streaming kernel
+    # the persistent kernel, batches on k_gemvr; and 37 blocks (K > 8192), where every M runs the
+    # streaming kernel
     (2000, 4352, 3), (3000, 4864, 8), (6390, 5888, 6), (2000, 7424, 5), (4100, 7936, 2), (100, 9472, 3)]
 
 
@@ -403,11 +402,14 @@ def test_gemv_fast_batch_invariance(N, K, M):
     assert ok, f"batch of M={M}: fp32 accumulators {worst:.3f} of the tolerance"
 
 
-# The any-K multi-row kernel (K > 6144, or a block count without another multi-row plan): one block per
-# wave and fewer blocks than waves, an odd part per wave, a ragged tile, 2..8 rows (both MFMA sets,
-# rows past M in a set), passes of 8 + remainder, and K past the two-workgroups-per-CU LDS plan.
-ANY_K_CASES = [(17, 8448, 2), (100, 12288, 3), (16, 10240, 5), (33, 32768, 8), (40, 49152, 6), (5, 7424, 4), (640, 5632, 8),
-               (300, 2816, 3), (48, 4352, 7), (8200, 6400, 2), (70, 8192, 10)]
+# Batches at long or unevenly divided K.  On k_gemvr (8 .. 64 blocks, K > 6144 or a block count without
+# another multi-row plan, and a one-row kernel in its order): an odd part per wave, a ragged tile, 2..8
+# rows (both MFMA sets, rows past M in a set), passes of 8 + remainder, four to seven waves that leave two
+# workgroups per CU and eight that do not (K = 12544 and 16384 at six and eight rows).  The last three do
+# not run it: K = 8448 a launch per row, K = 32768 and 49152 the streaming kernel.
+ANY_K_CASES = [(100, 12288, 3), (16, 10240, 5), (5, 7424, 4), (640, 5632, 8), (300, 2816, 3), (48, 4352, 7), (8200, 6400, 2),
+               (70, 8192, 10), (17, 8960, 2), (24, 10752, 4), (49, 9216, 3), (40, 12544, 6), (33, 16384, 8),
+               (17, 8448, 2), (33, 32768, 8), (40, 49152, 6)]
 
 
 @pytest.mark.parametrize("N,K,M", ANY_K_CASES)
