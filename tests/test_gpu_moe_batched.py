@@ -120,6 +120,21 @@ def test_batched_fast_more_experts_than_one_workgroup_routes(shared):
     _check_fast(y, sel, sw, X, BF16, rw, ex, sh, E, H, I, topk)
 
 
+@pytest.mark.parametrize("H,I,M,E,topk,shared", [(7168, 512, 2, 6, 2, True), (7168, 256, 8, 5, 2, False), (512, 8192, 2, 5, 2, False),
+                                                 (256, 7168, 5, 4, 3, True), (7168, 512, 9, 4, 1, True), (7168, 256, 3, 520, 2, False)])
+def test_batched_fast_union_of_wide_layers(H, I, M, E, topk, shared):
+    """H or I of 7168 / 8192: a leg that does not fit the small-batch kernel's plans, so a pass evaluates
+    the union of its rows' experts, every row on each (one or two rows: the down leg four tiles per
+    workgroup), routed in one workgroup or, for more than 512 experts, by the tail kernel."""
+    note(f"moe batched fast union H={H} I={I} M={M} E={E}")
+    rng = np.random.default_rng(H + I + M)
+    rw, ex, sh = _case(rng, E, H, I, BF16)
+    sh = sh if shared else None
+    X = qo.random_bf16(rng, (M, H), scale=0.05)
+    y, sel, sw = _run(BF16, rw, ex, sh, E, H, I, topk, X, "fast")
+    _check_fast(y, sel, sw, X, BF16, rw, ex, sh, E, H, I, topk)
+
+
 @pytest.mark.parametrize("M", [2, 4])
 def test_batched_fast_c2_shape(M):
     """Config-2 expert shape (6144 <-> 2048, top-8) over 32 experts, shared expert; two rows

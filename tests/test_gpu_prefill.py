@@ -70,6 +70,75 @@ def test_prefill_split_tiles(M, N, K):
     _check(raw, N, K, x, y, yf, f"M={M} N={N} K={K}")
 
 
+def _on_large_kernel(M, N, K):
+    """Whether the call has too many 64 x 32 tiles per CU for the split kernel (mirrors split_tile)."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return (M + 63) // 64 * ((N + 31) // 32) > (4 if K == 256 else 6) * cus and M > 32
+
+
+def _check_columns(raw, N, K, x, y, yf, what, n=40):
+    """_check on n columns, the first and the last among them."""
+    cols = np.unique(np.concatenate([[0, N - 1], np.random.default_rng(3).choice(N, n, replace=False)]))
+    sub = raw.reshape(N, -1)[cols].reshape(-1)
+    return _check(sub, len(cols), K, x, np.ascontiguousarray(y[:, cols]), np.ascontiguousarray(yf[:, cols]), what)
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 16500, 768), (257, 10001, 1280), (1000, 3300, 512), (129, 16417, 2304)])
+def test_prefill_large_kernel_ragged(M, N, K):
+    """The 128 x 256 kernel at ragged M and N with several super-blocks, odd numbers of them too."""
+    note(f"prefill large M={M} N={N} K={K}")
+    assert _on_large_kernel(M, N, K)
+    rng = np.random.default_rng(M + N + K)
+    raw = qo.random_q4k_blocks(rng, N * K // 256)
+    x = qo.random_bf16(rng, (M, K))
+    y, yf = _prefill(raw, N, K, x)
+    _check_columns(raw, N, K, x, y, yf, f"M={M} N={N} K={K}")
+
+
+def test_prefill_large_kernel_values():
+    """The 128 x 256 kernel on rows of very different magnitudes, zero rows and negative zeros, on blocks
+    with degenerate scales, with a workspace of a larger call, and again with the same bits; a changed
+    weight fails the gate."""
+    note("prefill large kernel values")
+    rng = np.random.default_rng(80)
+    M, N, K = 144, 16500, 768
+    assert _on_large_kernel(M, N, K)
+    raw = qo.random_q4k_blocks(rng, N * K // 256).reshape(-1, 144)
+    hdr = raw[:, 0:4].copy().view(np.uint16)
+    hdr[0::5, 0], hdr[1::5, 1], hdr[2::5, 0], hdr[3::5, :] = 0x0000, 0x0000, 0x0001, 0x8000
+    raw[:, 0:4] = hdr.view(np.uint8)
+    raw[4::7, 4:16], raw[5::7, 4:16] = 0xFF, 0x00
+    raw = raw.reshape(-1)
+    x = rng.standard_normal((M, K)) * 2.0 ** rng.choice([-120, -60, -20, 0, 7, 20, 60, 100], M)[:, None]
+    x[9], x[140] = 0.0, 0.0
+    x[11, ::7] *= 2.0 ** 40
+    x[12, ::3] = -0.0
+    x = qo.bf16_round_bits(x.astype(np.float32))
+    ws = dev.prefill_workspace(400, K, "cuda")
+    y, yf = _prefill(raw, N, K, x, ws)
+    _check_columns(raw, N, K, x, y, yf, "values")
+    assert np.all(yf[9] == 0.0) and np.all(yf[140] == 0.0)
+    y2, yf2 = _prefill(raw, N, K, x)
+    assert_bits_equal(y, y2, "again")
+    assert_bits_equal(yf.view(np.uint32), yf2.view(np.uint32), "again f32")
+    n = 5000                                        # one nibble of weight row n from 0 to 15
+    row = raw.reshape(N, -1)[n].copy()
+    row[0:4] = np.array([0x2000, 0x2000], np.uint16).view(np.uint8)
+    row[4:16] = qo.pack_scales_q4k([32] * 8, [1] * 8)
+    row[16 + 3] &= 0xF0
+    good = raw.reshape(N, -1).copy()
+    good[n] = row
+    bad = good.copy()
+    bad[n, 16 + 3] |= 0x0F
+    xc = x.copy()
+    xc[:, 3] = qo.bf16_round_bits(np.abs(qo.bf16_bits_to_f32(x)).max(1) * np.float32(4.0) + np.float32(1e-30))
+    wd, xf = qo.dequant_q4k(row).reshape(1, K), qo.bf16_bits_to_f32(xc)
+    _, fb = _prefill(bad.reshape(-1), N, K, xc)
+    assert not qo.tolerance_gate(wd, xf, np.ascontiguousarray(fb[:, n:n + 1]))[0], "the gate passed a corrupted weight"
+    _, fg = _prefill(good.reshape(-1), N, K, xc)
+    assert qo.tolerance_gate(wd, xf, np.ascontiguousarray(fg[:, n:n + 1]))[0]
+
+
 def test_prefill_activation_range():
     """Rows at very different magnitudes (2^-120 .. 2^100), an all-zero row, a row mixing huge
     and tiny values, negative zeros: the per-row power-of-two scaling keeps them exact."""
