@@ -240,6 +240,7 @@ __device__ __forceinline__ void ref_rows(const uint8_t* __restrict__ W, int64_t 
         const int nr = (int)(K / 16);       // whole runs
         // stage t's operands; runs past the last whole one repeat it (their products are not
         // read, or come from the partial path below)
+        // (16 r fits 32 bits: with one or two activation rows K < 2^31, see kMaxProductK)
         auto fetch = [&](Held<TYPE, C::G, C::kMul>& b, int t) {
             int r = t * C::RPS + un;
             r = r < nr ? r : nr - 1;
@@ -251,8 +252,8 @@ __device__ __forceinline__ void ref_rows(const uint8_t* __restrict__ W, int64_t 
             } else {
 #pragma unroll
                 for (int g = 0; g < C::G; ++g) {
-                    b.x[g][0] = load16_u2(xr[g] + 16 * (int64_t)r);
-                    b.x[g][1] = load16_u2(xr[g] + 16 * (int64_t)r + 8);
+                    b.x[g][0] = load16_u2(xr[g] + 16 * r);
+                    b.x[g][1] = load16_u2(xr[g] + 16 * r + 8);
                 }
             }
         };
@@ -635,35 +636,37 @@ struct RefGather {
     int64_t y_zstride;
 };
 
-__device__ __forceinline__ void ref_gather(const RefGather& ga, const uint8_t*& W, const uint16_t*& X, uint16_t*& Y,
-                                           float*& Yf) {
-    if (!ga.sel) return;
-    int z = blockIdx.z;
-    const uint8_t* alt = ga.W_alt;
-    if (z >= ga.nslots) {
-        z -= ga.nslots;
-        W = ga.W2;
-        alt = ga.W2_alt;
-        Y = ga.Y2;
+// The slot's pointers.  A macro: through a function's references the kernels lose their __restrict__
+// (6144 x 6144 Q4_K, M = 4: 38.6 -> 39.7 us; 2048 x 6144: 39.7 -> 42.9).
+#define AIPU_REF_GATHER(ga, W, X, Y, Yf)                     \
+    if (ga.sel) {                                            \
+        int z = blockIdx.z;                                  \
+        const uint8_t* alt = ga.W_alt;                       \
+        if (z >= ga.nslots) {                                \
+            z -= ga.nslots;                                  \
+            W = ga.W2;                                       \
+            alt = ga.W2_alt;                                 \
+            Y = ga.Y2;                                       \
+        }                                                    \
+        if (z < ga.topk) {                                   \
+            int e = ga.sel[z];                               \
+            e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e); \
+            W += (int64_t)e * ga.wstride;                    \
+        } else {                                             \
+            W = alt;                                         \
+        }                                                    \
+        X += (int64_t)z * ga.x_zstride;                      \
+        Y += (int64_t)z * ga.y_zstride;                      \
+        if (Yf) Yf += (int64_t)z * ga.y_zstride;             \
     }
-    if (z < ga.topk) {
-        int e = ga.sel[z];
-        e = e < 0 ? 0 : (e >= ga.E ? (int)ga.E - 1 : e);
-        W += (int64_t)e * ga.wstride;
-    } else {
-        W = alt;
-    }
-    X += (int64_t)z * ga.x_zstride;
-    Y += (int64_t)z * ga.y_zstride;
-    if (Yf) Yf += (int64_t)z * ga.y_zstride;
-}
 
 template <int TYPE, int MC, int RM>
-__global__ __launch_bounds__((RefCfg<MC, RM>::kThreads)) void k_gemv_ref(const uint8_t* W, int64_t N, int64_t K,
-                                                                         const uint16_t* X, int64_t M, uint16_t* Y,
-                                                                         float* Yf, int64_t ys, int R, RefGather ga) {
+__global__ __launch_bounds__((RefCfg<MC, RM>::kThreads)) void k_gemv_ref(const uint8_t* __restrict__ W, int64_t N, int64_t K,
+                                                                         const uint16_t* __restrict__ X, int64_t M,
+                                                                         uint16_t* __restrict__ Y, float* __restrict__ Yf,
+                                                                         int64_t ys, int R, RefGather ga) {
     extern __shared__ __align__(16) uint8_t s_ref[];
-    ref_gather(ga, W, X, Y, Yf);
+    AIPU_REF_GATHER(ga, W, X, Y, Yf)
     const int64_t m0 = (int64_t)blockIdx.y * MC;
     const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
     ref_rows<TYPE, MC, RM>(W, N, K, X + m0 * K, mcnt, Y + m0 * ys, Yf ? Yf + m0 * ys : nullptr, ys,
@@ -671,10 +674,11 @@ __global__ __launch_bounds__((RefCfg<MC, RM>::kThreads)) void k_gemv_ref(const u
 }
 
 template <int TYPE, int MC>
-__global__ __launch_bounds__(64) void k_gemv_ref_wave(const uint8_t* W, int64_t N, int64_t K, const uint16_t* X, int64_t M,
-                                                      uint16_t* Y, float* Yf, int64_t ys, RefGather ga) {
+__global__ __launch_bounds__(64) void k_gemv_ref_wave(const uint8_t* __restrict__ W, int64_t N, int64_t K,
+                                                      const uint16_t* __restrict__ X, int64_t M, uint16_t* __restrict__ Y,
+                                                      float* __restrict__ Yf, int64_t ys, RefGather ga) {
     __shared__ __align__(16) float s_x[2 * MC * kWaveChunk];
-    ref_gather(ga, W, X, Y, Yf);
+    AIPU_REF_GATHER(ga, W, X, Y, Yf)
     const int64_t m0 = (int64_t)blockIdx.y * MC;
     const int mcnt = (int)((M - m0) < MC ? (M - m0) : MC);
     ref_wave<TYPE, MC>(W, N, K, X + m0 * K, mcnt, Y + m0 * ys, Yf ? Yf + m0 * ys : nullptr, ys, (int64_t)blockIdx.x * 64, s_x);
@@ -768,6 +772,10 @@ int ref_rows_per_wg(int64_t rows, int cap) {
 // along x fit 32 bits).
 constexpr int64_t kMaxRows = 1LL << 26, kMaxPasses = 65535;
 
+// Longer rows run the kernel of three and more activation rows, whose offsets into them are 64-bit (with
+// 64-bit offsets the kernel of one row took 23.4 us at 6144 x 6144, 22.5 without); a run's index is 32-bit.
+constexpr int64_t kMaxProductK = (1LL << 31) - 1, kMaxRefK = (1LL << 35) - 1;
+
 // Calls fn(n0, n, m0, m) for pieces of at most kMaxRows rows and kMaxPasses passes.
 template <class F>
 hipError_t for_pieces(int64_t N, int64_t M, int mc, F fn) {
@@ -855,7 +863,8 @@ bool ref_wave_wins(int type, int64_t rows, int64_t M, int64_t K) {
     const int per = (int)(rows / device_cu_count() < 1 << 20 ? rows / device_cu_count() : 1 << 20);
     const int i = M >= 5 ? 3 : M >= 3 ? 2 : (int)M - 1;
     if (type == T_Q4_K) {
-        const int at[4] = {K <= 256 ? 104 : 130, K <= 512 ? 64 : 97, K <= 512 ? 130 : 194, K <= 256 ? 208 : K <= 512 ? 256 : 288};
+        const int at[4] = {K <= 256 ? 104 : 130, K <= 512 ? 64 : 97, K <= 256 ? 130 : K <= 512 ? 156 : 194,
+                           K <= 256 ? 208 : K <= 512 ? 256 : 288};
         return per >= at[i];
     }
     if (type == T_Q6_K) {
@@ -865,7 +874,7 @@ bool ref_wave_wins(int type, int64_t rows, int64_t M, int64_t K) {
     if (i == 0) return K <= 256 ? per >= 120 : type != T_Q8_0 && K <= 2048 && per >= 130 && per < (K <= 1024 ? 400 : 256);
     if (i == 1) return per >= (K <= 512 ? 64 : type != T_Q8_0 && K >= 4096 ? 130 : 97);
     if (i == 2) return per >= (K <= 512 ? 130 : K > 8192 ? 256 : 194);
-    return K <= 256 ? per >= 232 : K <= 512 && per >= 380;
+    return K <= 256 ? per >= 300 : K <= 512 && per >= 380;
 }
 
 template <int TYPE>
@@ -877,13 +886,14 @@ hipError_t run_ref_type(const RefCall& c) {
         return M == 2 ? run_ref_wave<TYPE, 2>(c) : run_ref_wave<TYPE, 1>(c);
     }
     if (M >= 5) return run_ref<TYPE, 8, 32>(c);
-    if (M >= 3) return run_ref<TYPE, 4, 32>(c);
+    if (M >= 3 || c.K > kMaxProductK) return run_ref<TYPE, 4, 32>(c);
     if (M == 2) return run_ref<TYPE, 2, 32>(c);
     if (c.N * c.nslots <= 32 * (int64_t)device_cu_count()) return run_ref<TYPE, 1, 32>(c);
     return run_ref<TYPE, 1, 64>(c);
 }
 
 hipError_t run_ref_any(int type, const RefCall& c) {
+    if (c.K > kMaxRefK) return hipErrorInvalidValue;
     switch (type) {
         case T_Q4_K: return run_ref_type<T_Q4_K>(c);
         case T_Q6_K: return run_ref_type<T_Q6_K>(c);
@@ -912,7 +922,7 @@ hipError_t launch_gemv_ref(int type, const void* w, int64_t N, int64_t K, const 
 
 hipError_t launch_gemv_ref_tiles(const aipu_tile_desc* tiles, int n_tiles, int64_t K, const uint16_t* x, int64_t M,
                                  uint16_t* y, float* y_f32, int64_t ys, hipStream_t st) {
-    if (n_tiles < 1 || n_tiles > AIPU_MAX_TILES || M < 1) return hipErrorInvalidValue;
+    if (n_tiles < 1 || n_tiles > AIPU_MAX_TILES || M < 1 || K > kMaxRefK) return hipErrorInvalidValue;
     // tiles of so many rows that the one-wave kernel is faster run by themselves, the others in one launch
     aipu_tile_desc rest[AIPU_MAX_TILES];
     int n_rest = 0;
@@ -967,7 +977,7 @@ hipError_t launch_gemv_ref_tiles(const aipu_tile_desc* tiles, int n_tiles, int64
         return flush();
     };
     if (M >= 5) return run(RefCfg<8, 32>{}, k_gemv_ref_tiles<8, 32>, 8, 32);
-    if (M >= 3) return run(RefCfg<4, 32>{}, k_gemv_ref_tiles<4, 32>, 4, 32);
+    if (M >= 3 || K > kMaxProductK) return run(RefCfg<4, 32>{}, k_gemv_ref_tiles<4, 32>, 4, 32);
     if (M == 2) return run(RefCfg<2, 32>{}, k_gemv_ref_tiles<2, 32>, 2, 32);
     if (rows <= 32 * (int64_t)device_cu_count()) return run(RefCfg<1, 32>{}, k_gemv_ref_tiles<1, 32>, 1, 32);
     return run(RefCfg<1, 64>{}, k_gemv_ref_tiles<1, 64>, 1, 64);

@@ -237,9 +237,9 @@ def test_gemv_ref_row_split(t, N, K, M):
 WAVE_CASES = [
     (qo.GGML_Q4_K, 40001, 256, 1), (qo.GGML_Q4_K, 25001, 768, 2), (qo.GGML_Q4_K, 50001, 512, 3), (qo.GGML_Q4_K, 37003, 256, 9),
     (qo.GGML_Q6_K, 17001, 1024, 1), (qo.GGML_Q6_K, 17030, 512, 2), (qo.GGML_Q6_K, 34001, 512, 4), (qo.GGML_Q6_K, 17001, 768, 1),
-    (qo.GGML_Q8_0, 31001, 192, 1), (qo.GGML_Q8_0, 25002, 576, 2), (qo.GGML_Q8_0, 50001, 640, 4), (qo.GGML_Q8_0, 60001, 64, 8),
+    (qo.GGML_Q8_0, 31001, 192, 1), (qo.GGML_Q8_0, 25002, 576, 2), (qo.GGML_Q8_0, 50001, 640, 4), (qo.GGML_Q8_0, 78001, 64, 8),
     (qo.GGML_F16, 34001, 320, 1), (qo.GGML_F16, 113001, 2048, 2), (qo.GGML_F16, 34001, 448, 3), (30, 34001, 832, 1),
-    (30, 60001, 128, 8),
+    (30, 78001, 128, 8),
 ]
 
 
