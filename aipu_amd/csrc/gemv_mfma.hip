@@ -1191,9 +1191,12 @@ hipError_t launch_gemv_mfma(const void* w, int64_t N, int64_t K, const uint16_t*
         uint16_t* ym = y + m0 * ystride;
         float* yfm = y_f32 ? y_f32 + m0 * ystride : nullptr;
         if (left >= 2 && canon1) {
-            // two rows on the one-row kernel (dense: where neither the dense kernel nor k_gemvs serves the
-            // shape; 512 x 4352 3.8 us there and 4.4 on k_gemvr)
-            if (left == 2 && gemv_persist2_supported(N, K) && (!dense || (!small && !gemv_persist_m_supported(N, K, 2, true)))) {
+            // two rows on the one-row kernel.  Dense, where neither the dense kernel nor k_gemvs serves the
+            // shape: where it beats k_gemvr (512 x 4352 3.8 and 4.4 us, 6144 x 5632 6.6 and 7.9; 4096 x 2816 4.5
+            // and 3.9, 8192 x 2816 6.5 and 5.3)
+            const int64_t cus = device_cu_count();
+            const bool dense2 = !small && !gemv_persist_m_supported(N, K, 2, true) && (N <= 8 * cus || (K > 4096 && N > 16 * cus));
+            if (left == 2 && gemv_persist2_supported(N, K) && (!dense || dense2)) {
                 const hipError_t e = launch_gemv_persist2(W, N, K, xm, ym, yfm, ystride, st);
                 if (e != hipSuccess) return e;
                 m0 += 2;
