@@ -686,7 +686,7 @@ __global__ __launch_bounds__(64) void k_gemv_ref_wave(const uint8_t* __restrict_
 
 // A tile sequence of mixed types in one launch: workgroup g belongs to the last tile whose wg0 is
 // at most g.  The tiles' launches one after the other would each take a whole chain (24 tiles of
-// 256 rows, K = 6144: 1.82 ms as 24 launches of the earlier kernel, one launch 27 us).
+// 256 rows, K = 6144, M = 1: 1.82 ms as 24 launches of the earlier kernel, one launch 35 us).
 struct RefTile {
     const uint8_t* w;
     int64_t row0, nrows;
@@ -827,7 +827,7 @@ hipError_t run_ref(const RefCall& c) {
 template <int TYPE, int MC>
 hipError_t run_ref_wave(const RefCall& c) {
     // 16-bit rows at two activation rows: four waves per CU where more would thrash the rows' lines (200000 x
-    // 6144: 661 -> 578 us; 72000 x 6144, whose waves all fit, 198 -> 273)
+    // 6144: 661 -> 570 us; 72000 x 6144, whose waves all fit, 198 -> 273)
     const bool few = (TYPE == T_F16 || TYPE == T_BF16) && MC == 2 && c.K >= 2048 &&
                      c.N * c.nslots * ((c.M + MC - 1) / MC) >= 440 * (int64_t)device_cu_count();
     const int pad = few ? 40 * 1024 - 2 * MC * kWaveChunk * 4 : 0;
@@ -853,11 +853,11 @@ bool ref_wave_takes(int type, const RefCall& c) {
 // activation rows).  ref_rows takes a time that grows with the rows once every CU has a workgroup, in
 // steps of 32 rows per CU; the one-wave kernel takes the same time up to 64 rows per SIMD.  The lines
 // cross at these rows per CU, earlier where K is short and ref_rows' stages are few.  Q4_K, K = 6144,
-// ref_rows > one wave: M = 1, 32768 / 65536 / 154880 rows 62 > 74 / 115 > 75 / 282 > 141 us; M = 2, 24576 /
-// 32768 / 65536 rows 90 > 100 / 118 > 101 / 230 > 105 us; M = 4, 49152 / 65536 rows 156 > 172 / 208 > 177 us;
-// M = 8, 65536 / 98304 rows 262 > 300 / 389 > 340 us.  Q8_0 and the 16-bit types, whose rows the one-wave
-// kernel reads 68 or 128 bytes at a time, stay on ref_rows at M = 1 and M = 8 (Q8_0: 131072 rows 345 and
-// 415 us at M = 1, 154880 rows 616 and 735 us at M = 8), but for a short K, and 16 bits
+// ref_rows > one wave: M = 1, 32768 / 65536 / 154880 rows 61 > 74 / 114 > 74 / 282 > 175 us; M = 2, 24576 /
+// 32768 / 65536 rows 89 > 100 / 116 > 99 / 227 > 102 us; M = 4, 49152 / 65536 rows 155 > 172 / 204 > 171 us;
+// M = 8, 65536 / 98304 rows 267 > 300 / 412 > 327 us.  Q8_0 and the 16-bit types, whose rows the one-wave
+// kernel reads 68 or 128 bytes at a time, stay on ref_rows at M = 1 and M = 8 (Q8_0: 131072 rows 344 and
+// 415 us at M = 1, 154880 rows 643 and 735 us at M = 8), but for a short K, and 16 bits
 // from 130 rows per CU to 256 or 400 at M = 1 and K <= 2048 (200000 x 1024: 72 and 97 us).
 bool ref_wave_wins(int type, int64_t rows, int64_t M, int64_t K) {
     const int per = (int)(rows / device_cu_count() < 1 << 20 ? rows / device_cu_count() : 1 << 20);

@@ -414,7 +414,7 @@ ANY_K_CASES = [(100, 12288, 3), (16, 10240, 5), (5, 7424, 4), (640, 5632, 8), (3
 
 @pytest.mark.parametrize("N,K,M", ANY_K_CASES)
 def test_gemv_fast_any_k_rows(N, K, M):
-    note(f"gemv fast any K N={N} K={K} M={M}")
+    note(f"gemv fast long K N={N} K={K} M={M}")
     rng = np.random.default_rng(17 * N + K + M)
     raw = qo.random_q4k_blocks(rng, N * K // 256)
     x = qo.random_bf16(rng, (M, K))
@@ -431,7 +431,7 @@ def test_gemv_fast_any_k_rows(N, K, M):
 @pytest.mark.parametrize("N,K,M", [(512, 4352, 2), (100, 2816, 2), (6144, 2816, 10), (16384, 4352, 2)])
 def test_gemv_dense_two_rows_without_dense_kernel(N, K, M):
     """Dense mode at block counts without a dense kernel: two rows (or two left of a batch) on the one-row
-    kernel or the any-K kernel, every row with its one-row bits."""
+    kernel or k_gemvr, every row with its one-row bits."""
     note(f"gemv dense two rows N={N} K={K} M={M}")
     rng = np.random.default_rng(N + K + M)
     raw = qo.random_q4k_blocks(rng, N * K // 256)

@@ -226,7 +226,8 @@ def test_batched_fast_two_row_pass_equals_one_row_pass(H, topk, shared):
 def test_batched_fast_slot_lists(M, E, topk, shared):
     """The slot lists of a pass at their limits: every row on every expert (four slots each, the
     last one half empty at seven rows), fewer experts than rows, a leftover row, routing outside
-    the one-workgroup kernel, and more than eight and sixteen experts per row; within the fast-mode bound, and every row equal to a two-row batch."""
+    the one-workgroup kernel, and more than eight and sixteen experts per row; within the fast-mode
+    bound, and every row equal to a two-row batch."""
     H, I = 512, 256
     note(f"moe batched fast slot lists M={M} E={E} topk={topk} shared={shared}")
     rng = np.random.default_rng(31 * M + E)
